@@ -1,0 +1,69 @@
+"""The leaf-network kernels at the edges of their tiles, through the C ABI.
+
+Float32: bit-identical to the oracle's CPU loop at every tile size the
+dispatch takes (few, some and many rows), with inputs, hidden widths and heads
+that fill no tile, no 16-byte run and no k tile, from buffers that 16-byte
+loads may not read, and with infinite weights behind zero inputs.
+"""
+import sys
+
+import numpy as np
+import pytest
+
+import oracle as O
+import warchest_wave as ww
+from test_zz_no_alloc import Hip
+
+pytestmark = pytest.mark.gpu
+
+
+def say(msg):
+    print(msg, flush=True)
+    sys.stdout.flush()
+
+
+def forward_on_device(ex, v, x, heads, offset):
+    """mlp_noalloc with both buffers `offset` floats past a 256-byte boundary."""
+    hip = Hip()
+    rows = x.shape[0]
+    xd, od = hip.alloc((x.size + offset) * 4), hip.alloc((rows * heads + offset) * 4)
+    try:
+        hip.to_dev(xd + 4 * offset, x)
+        ex.mlp_noalloc(v, rows, xd + 4 * offset, od + 4 * offset)
+        out = np.zeros((rows, heads), np.float32)
+        hip.to_host(out, od + 4 * offset)
+        return out
+    finally:
+        hip.free(xd)
+        hip.free(od)
+
+
+# rows x outputs cross the line between the 16-, 32- and 64-wide tiles
+@pytest.mark.parametrize("inputs,hidden,layers,heads,rows,offset", [
+    (101, 50, 2, 7, 1, 0), (130, 64, 1, 1, 17, 1), (512, 384, 3, 22, 64, 0), (97, 130, 2, 567, 333, 3),
+    (160, 384, 2, 33, 1500, 2), (132, 384, 1, 65, 5500, 0), (31, 391, 1, 22, 6001, 1)])
+def test_float32_net_edges(inputs, hidden, layers, heads, rows, offset):
+    say(f"case float32 net: {rows} rows, {inputs} -> {layers}x{hidden} -> {heads}, buffers + {offset} floats")
+    net = ww.synth_weights(ww.mlp_dims(inputs, hidden, layers, heads, pool=8), seed=rows)
+    x = ww.synth_features(rows, inputs, seed=rows + 1)
+    ex = ww.Executor(0, ww.WC_PRECISE)
+    got = forward_on_device(ex, ex.publish(net), x, heads, offset)
+    ex.close()
+    keys = np.tile(np.arange(heads, dtype=np.uint32), (rows, 1))
+    np.testing.assert_array_equal(got, O.mlp(x, keys, net, O.NET_F32))
+
+
+def test_float32_net_skips_zero_inputs_of_infinite_weights():
+    say("case float32 net: infinite and NaN weights behind zero and non-zero inputs")
+    net = ww.synth_weights(ww.mlp_dims(36, 40, 2, 5, pool=8), seed=3)
+    x = ww.synth_features(50, 36, seed=4)
+    x[:25, 7] = 0.0
+    net.w[7 * 40 + 11] = np.inf
+    net.w[7 * 40 + 12] = np.nan
+    ex = ww.Executor(0, ww.WC_PRECISE)
+    got = ex.mlp(ex.publish(net), x, heads=5)
+    ex.close()
+    keys = np.tile(np.arange(5, dtype=np.uint32), (50, 1))
+    want = O.mlp(x, keys, net, O.NET_F32)
+    assert np.isfinite(want[:25]).all() and not np.isfinite(want[25:]).all()
+    np.testing.assert_array_equal(got, want)

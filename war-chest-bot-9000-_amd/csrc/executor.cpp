@@ -315,9 +315,8 @@ uint64_t Executor::publish(const NetShape& ns, const std::vector<uint32_t>& dims
     // compensated pair (hi and lo planes).
     const size_t esz = precision_ == WC_PRECISE ? 4 : precision_ == WC_F16X ? 4 : 2;
     // Layout: matrices (as stored for the arithmetic), then f32 biases, then
-    // the two-tower readout weight. The exact net keeps the source layout; the
-    // MFMA net stores each matrix as the GEMM's B operand (one row per output,
-    // K-contiguous), fragment-major with gemm_rows(N) zero-padded rows.
+    // the two-tower readout weight. Both nets store one K-contiguous row per
+    // output; the MFMA net fragment-major with gemm_rows(N) zero-padded rows.
     std::vector<size_t> moff;
     size_t at = 0;
     auto stored_bytes = [&](const Mat& m) {
@@ -333,9 +332,8 @@ uint64_t Executor::publish(const NetShape& ns, const std::vector<uint32_t>& dims
     at = align256(at + nb * 4);
     const size_t roff = at;  // readout weight (two-tower), f32
     if (tower) at = align256(at + size_t(ns.hidden) * 4);
-    // Staging for f32 -> 16-bit conversion on the device.
-    const size_t stage = precision_ == WC_PRECISE ? 0 : at;
-    const size_t total = at + (precision_ == WC_PRECISE ? 0 : nw * 4);
+    // Staging for the conversion to the stored layout on the device.
+    const size_t stage = at, total = at + nw * 4;
     void* mem = nullptr;
     if (hipMalloc(&mem, total) != hipSuccess) {
         *err = "hipMalloc of the weight bank failed";
@@ -344,15 +342,24 @@ uint64_t Executor::publish(const NetShape& ns, const std::vector<uint32_t>& dims
     char* base = (char*)mem;
     bool okc = hipMemcpyAsync(base + boff, b, nb * 4, hipMemcpyHostToDevice, stream_) == hipSuccess;
     size_t src = 0;
+    okc = okc && hipMemcpyAsync(base + stage, w, nw * 4, hipMemcpyHostToDevice, stream_) == hipSuccess;
     if (precision_ == WC_PRECISE) {
+        // (as integers: the comparison vectorises)
+        const uint32_t inf = 0x7f800000u;
+        uint32_t bad = 0;
+        for (size_t k = 0; k < nw; k++) {
+            uint32_t u;
+            std::memcpy(&u, w + k, 4);
+            bad |= (u & inf) == inf ? 1u : 0u;
+        }
+        bank.skip = bad != 0;
         for (size_t k = 0; k < mats.size(); k++) {
-            const size_t n = mats[k].k * mats[k].n;
-            okc = okc && hipMemcpyAsync(base + moff[k], w + src, n * 4, hipMemcpyHostToDevice, stream_) == hipSuccess;
-            src += n;
+            launch_rows((const float*)(base + stage) + src, (float*)(base + moff[k]), (uint32_t)mats[k].n,
+                        (uint32_t)mats[k].k, !mats[k].head, stream_);
+            src += mats[k].k * mats[k].n;
         }
     } else {
         okc = okc && hipMemsetAsync(base, 0, mats_end, stream_) == hipSuccess;  // row padding
-        okc = okc && hipMemcpyAsync(base + stage, w, nw * 4, hipMemcpyHostToDevice, stream_) == hipSuccess;
         for (size_t k = 0; k < mats.size(); k++) {
             const size_t n = mats[k].k * mats[k].n;
             // Trunk and tower matrices are [K x N] (B row n = source column n);
@@ -423,7 +430,7 @@ bool Executor::upload(const WaveHost& w, const NetBank& bank, uint32_t slot, std
         size_t node_meta, nc, legal_value, draw_to, draw_p, reach_base, vals_base, rev_src, rev_cell, rvd_src, rvd_p,
             row_node, row_cfg_off, row_cfg, cfg_emb, pub_raw, term_node, term_util, roots, carried, exit_node,
             exit_coff, exit_reach, trees, units, bt[2], rt[2], dc[2], bl[2], rl[2], cv[2], lr[2], pg[2], twb[2], twu[2], cfg_priv,
-            unit_term, tb[2], tr[2], tc[2], rc[2], rp[2], head_tile_n, cp[2], card_feat, row_job, cfg_job, cfg_owner;
+            unit_term, tb[2], tr[2], tc[2], rc[2], rp[2], head_tile_n, hb[2], cp[2], card_feat, row_job, cfg_job, cfg_owner;
     } o;
     o.node_meta = blob.put(w.node_meta);
     o.nc = blob.put(w.node_nc);
@@ -474,6 +481,7 @@ bool Executor::upload(const WaveHost& w, const NetBank& bank, uint32_t slot, std
         plan[p] = plan_chain(w.head_rb_n[p].data(), (uint32_t)w.head_rb_n[p].size(), w.net.heads, cus_);
         if (!check_chain_plan(plan[p], w.head_rb_n[p].data(), (uint32_t)w.head_rb_n[p].size(), w.net.heads, err))
             return false;
+        o.hb[p] = blob.put(w.head_rb_n[p]);
         o.cp[p] = blob.put(plan[p]);
         chain_npass_[p] = (uint32_t)plan[p].size();
     }
@@ -605,7 +613,10 @@ bool Executor::upload(const WaveHost& w, const NetBank& bank, uint32_t slot, std
     }
     d.unit_term = (const uint32_t*)(T + o.unit_term);
     head_tile_n_ = (const uint32_t*)(T + o.head_tile_n);
-    for (int p = 0; p < 2; p++) chain_plan_[p] = (const ChainPass*)(T + o.cp[p]);
+    for (int p = 0; p < 2; p++) {
+        chain_plan_[p] = (const ChainPass*)(T + o.cp[p]);
+        head_rb_n_[p] = (const uint32_t*)(T + o.hb[p]);
+    }
     for (int p = 0; p < 2; p++) {
         top_back_dev_[p] = (const BackRec*)(T + o.tb[p]);
         top_reach_dev_[p] = (const ReachRec*)(T + o.tr[p]);
@@ -736,7 +747,8 @@ ChainNet chain_net(const NetBank& bank) {
 }
 
 void Executor::run_mlp(const NetBank& bank, uint32_t rows, const void* x, std::vector<hipEvent_t>* marks,
-                       const uint32_t* head_tile_n, const ChainPass* plan, uint32_t npass, const float* part) {
+                       const uint32_t* head_tile_n, const ChainPass* plan, uint32_t npass, const float* part,
+                       const uint32_t* head_rb_n) {
     const NetShape& ns = bank.ns;
     auto mark = [&]() {
         if (marks) {
@@ -762,7 +774,7 @@ void Executor::run_mlp(const NetBank& bank, uint32_t rows, const void* x, std::v
         void* out = H_[l & 1];
         if (precision_ == WC_PRECISE)
             launch_dense_exact((const float*)in, k, (const float*)bank.W[l], bank.B[l], ns.hidden, (float*)out, rows,
-                               stream_);
+                               bank.skip, stream_);
         else
             launch_gemm16(precision_, in, k, bank.W[l], bank.B[l], ns.hidden, out, rows, true, true, stream_);
         mark();
@@ -771,7 +783,7 @@ void Executor::run_mlp(const NetBank& bank, uint32_t rows, const void* x, std::v
     }
     if (precision_ == WC_PRECISE)
         launch_head_exact((const float*)in, ns.hidden, (const float*)bank.Whead, bank.bhead, ns.heads, head_out_,
-                          rows, stream_);
+                          rows, stream_, head_rb_n);
     else
         launch_gemm16(precision_, in, ns.hidden, bank.Whead, bank.bhead, ns.heads, head_out_, rows, false, false,
                       stream_, head_tile_n);
@@ -791,7 +803,7 @@ void Executor::run_tower_private(const NetBank& bank) {
         void* out = P_[l & 1];
         if (precision_ == WC_PRECISE)
             launch_dense_exact((const float*)in, k, (const float*)bank.PW[l], bank.PB[l], ns.hidden, (float*)out,
-                               ncfg_, stream_);
+                               ncfg_, bank.skip, stream_);
         else
             launch_gemm16(precision_, in, k, bank.PW[l], bank.PB[l], ns.hidden, out, ncfg_, true, true, stream_);
         in = out;
@@ -808,7 +820,7 @@ void Executor::run_tower(const NetBank& bank, uint32_t rows, int traverser) {
         void* out = H_[l & 1];
         if (precision_ == WC_PRECISE)
             launch_dense_exact((const float*)in, k, (const float*)bank.W[l], bank.B[l], ns.hidden, (float*)out, rows,
-                               stream_);
+                               bank.skip, stream_);
         else
             launch_gemm16(precision_, in, k, bank.W[l], bank.B[l], ns.hidden, out, rows, true, true, stream_);
         in = out;
@@ -847,7 +859,8 @@ void Executor::leaf_net(const NetBank& bank, int q) {
     else if (bank.ns.kind == MODEL_TWO_TOWER)
         run_tower(bank, dev_.rows, q);
     else
-        run_mlp(bank, dev_.rows, Xq_[q], nullptr, head_tile_n_, chain_plan_[q], chain_npass_[q], S_[q]);
+        run_mlp(bank, dev_.rows, Xq_[q], nullptr, head_tile_n_, chain_plan_[q], chain_npass_[q], S_[q],
+                head_rb_n_[q]);
 }
 
 // Top regions' values bottom-up, one launch per run of the wave's plan: one

@@ -24,8 +24,11 @@ struct NetBank {
     NetShape ns;
     int precision = 0;
     void* mem = nullptr;  // one device allocation holding every matrix and bias
+    // Matrices as stored for the arithmetic: the MFMA operands, or in float32
+    // one K-contiguous row per output.
     const void* W[16] = {};
     const float* B[16] = {};
+    bool skip = false;  // float32: some weight is not finite, so zero inputs' terms must be left out
     const void* Whead = nullptr;
     const float* bhead = nullptr;
     // Two-tower net: W/B hold the public tower; the private tower, the readout
@@ -217,7 +220,8 @@ class Executor {
     // part: the first layer's precomputed product over the query inputs'
     // fixed columns (S_), or null.
     void run_mlp(const NetBank& bank, uint32_t rows, const void* x, std::vector<hipEvent_t>* marks,
-                 const uint32_t* head_tile_n, const ChainPass* plan, uint32_t npass, const float* part = nullptr);
+                 const uint32_t* head_tile_n, const ChainPass* plan, uint32_t npass, const float* part = nullptr,
+                 const uint32_t* head_rb_n = nullptr);
     bool ensure(void** p, size_t* cap, size_t need, std::string* err);
     bool ensure_pinned(uint8_t** p, size_t* cap, size_t need, std::string* err);
 
@@ -265,6 +269,7 @@ class Executor {
     const uint32_t* top_reach_chunk_dev_[2] = {};  // chunk bounds of the fused reach launches
     const uint32_t* top_reach_par_dev_[2] = {};    // and the shallower rows each chunk computes
     const uint32_t* head_tile_n_ = nullptr;  // head width per 128-row tile (device copy)
+    const uint32_t* head_rb_n_[2] = {};      // head width per 16-row block and traverser (device copies)
     const ChainPass* chain_plan_[2] = {};    // fused value net passes per traverser (device copies)
     uint32_t chain_npass_[2] = {0, 0};
     const ChainPass* mlp_plan_ = nullptr;    // the same for mlp_forward's rows

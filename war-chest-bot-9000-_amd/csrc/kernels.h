@@ -133,12 +133,20 @@ void launch_gather_carry(const WaveDev& w, const float* reach, int slot, hipStre
 void launch_collect_root(const WaveDev& w, int root, int player, hipStream_t s);
 
 // Leaf MLP.
-// Exact float32 dense ReLU layer in the CPU loop order: Y = relu(X W + b), W [K x N] row-major.
-void launch_dense_exact(const float* X, uint32_t K, const float* W, const float* b, uint32_t N, float* Y,
-                        uint32_t rows, hipStream_t s);
-// Exact float32 head: out[r, k] = b[k] + sum_j Wh[k, j] H[r, j], Wh [heads x hidden].
+// Exact float32 layers (exact.hip), in the CPU loop order; Wt holds one
+// K-contiguous row per output.
+// launch_rows lays a weight matrix out so: from [K x N] when transposed, else
+// from [N x K].
+void launch_rows(const float* src, float* dst, uint32_t N, uint32_t K, bool transposed, hipStream_t s);
+// Y = relu(X Wt^T + b). skip: leave out zero inputs' terms, as the CPU loop
+// does (needed for a bank with an infinite or NaN weight, NetBank::skip).
+void launch_dense_exact(const float* X, uint32_t K, const float* Wt, const float* b, uint32_t N, float* Y,
+                        uint32_t rows, bool skip, hipStream_t s);
+// The head: out[r, k] = b[k] + sum_j Wh[k, j] H[r, j], Wh [heads x hidden].
+// rb_n (optional, one entry per 16 rows) bounds the columns each row block
+// needs; columns past every bound of a tile are not computed.
 void launch_head_exact(const float* H, uint32_t hidden, const float* Wh, const float* bh, uint32_t heads,
-                       float* out, uint32_t rows, hipStream_t s);
+                       float* out, uint32_t rows, hipStream_t s, const uint32_t* rb_n = nullptr);
 // MFMA GEMM: Y[M, N] = act(X[M, K] Wt[N, K]^T + b); 16-bit fragment-major
 // operands (X with gemm_rows(M) rows, Wt with gemm_rows(N) rows), f32
 // accumulate. precision WC_F16 / WC_BF16; relu selects the activation; out16

@@ -1099,51 +1099,6 @@ void launch_collect_root(const WaveDev& w, int root, int player, hipStream_t s) 
     hipLaunchKernelGGL(k_collect_root, dim3(w.ntrees), dim3(BLOCK), 0, s, w, root, player);
 }
 
-// ------------------------------------------------------- leaf MLP (exact)
-
-// y[r, j] = relu(sum_p x[r, p] W[p, j] + b[j]): per output, from zero over
-// ascending inputs, zero inputs skipped (engine/src/net.rs:102-122).
-__global__ void k_dense_exact(const float* X, uint32_t K, const float* W, const float* b, uint32_t N, float* Y,
-                              uint32_t rows) {
-    size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (size_t)rows * N) return;
-    uint32_t r = (uint32_t)(i / N), j = (uint32_t)(i % N);
-    const float* x = X + (size_t)r * K;
-    float acc = 0.0f;
-    for (uint32_t p = 0; p < K; p++) {
-        float a = x[p];
-        if (a == 0.0f) continue;
-        acc += a * W[(size_t)p * N + j];
-    }
-    float v = acc + b[j];
-    Y[i] = v > 0.0f ? v : 0.0f;
-}
-
-void launch_dense_exact(const float* X, uint32_t K, const float* W, const float* b, uint32_t N, float* Y,
-                        uint32_t rows, hipStream_t s) {
-    size_t n = (size_t)rows * N;
-    if (n) hipLaunchKernelGGL(k_dense_exact, dim3(grid_for(n)), dim3(BLOCK), 0, s, X, K, W, b, N, Y, rows);
-}
-
-// out[r, k] = b[k] + sum_j Wh[k, j] H[r, j] (Net::values, engine/src/net.rs:844-853).
-__global__ void k_head_exact(const float* H, uint32_t hidden, const float* Wh, const float* bh, uint32_t heads,
-                             float* out, uint32_t rows) {
-    size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (size_t)rows * heads) return;
-    uint32_t r = (uint32_t)(i / heads), k = (uint32_t)(i % heads);
-    const float* h = H + (size_t)r * hidden;
-    const float* wr = Wh + (size_t)k * hidden;
-    float v = bh[k];
-    for (uint32_t j = 0; j < hidden; j++) v += wr[j] * h[j];
-    out[i] = v;
-}
-
-void launch_head_exact(const float* H, uint32_t hidden, const float* Wh, const float* bh, uint32_t heads,
-                       float* out, uint32_t rows, hipStream_t s) {
-    size_t n = (size_t)rows * heads;
-    if (n) hipLaunchKernelGGL(k_head_exact, dim3(grid_for(n)), dim3(BLOCK), 0, s, H, hidden, Wh, bh, heads, out, rows);
-}
-
 // ------------------------------------------------------- leaf MLP (MFMA)
 
 

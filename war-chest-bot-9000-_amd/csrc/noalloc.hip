@@ -117,7 +117,8 @@ bool Executor::mlp_forward_noalloc(uint64_t version, uint32_t rows, const float*
         uint32_t k = ns.in;
         for (uint32_t l = 0; l < ns.layers; l++) {
             float* o = (float*)(base + (l & 1 ? o_h1 : o_h0));
-            launch_dense_exact(in, k, (const float*)bank->W[l], bank->B[l], ns.hidden, o, rows, s);
+            launch_dense_exact(in, k, (const float*)bank->W[l], bank->B[l], ns.hidden, o, rows, bank->skip,
+                               s);
             in = o;
             k = ns.hidden;
         }
