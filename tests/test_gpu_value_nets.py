@@ -67,3 +67,20 @@ def test_float32_net_skips_zero_inputs_of_infinite_weights():
     want = O.mlp(x, keys, net, O.NET_F32)
     assert np.isfinite(want[:25]).all() and not np.isfinite(want[25:]).all()
     np.testing.assert_array_equal(got, want)
+
+
+# one pass per row block, several blocks per pass with a short last one, full passes; buffers off 16 bytes
+@pytest.mark.parametrize("precision", [ww.WC_F16, ww.WC_BF16])
+@pytest.mark.parametrize("inputs,hidden,layers,heads,rows,offset", [
+    (512, 384, 3, 567, 1, 0), (32, 32, 1, 1, 17, 1), (512, 384, 3, 22, 250, 3), (96, 352, 2, 130, 4113, 0),
+    (480, 128, 8, 64, 9000, 2), (512, 384, 3, 64, 32000, 0)])
+def test_fused_net_from_rows_equals_the_planned_passes(precision, inputs, hidden, layers, heads, rows, offset):
+    say(f"case fused net {precision}: {rows} rows, {inputs} -> {layers}x{hidden} -> {heads}, buffers + {offset} floats")
+    net = ww.synth_weights(ww.mlp_dims(inputs, hidden, layers, heads, pool=8), seed=rows)
+    x = ww.synth_features(rows, inputs, seed=rows + 1)
+    ex = ww.Executor(0, precision)
+    v = ex.publish(net)
+    got = forward_on_device(ex, v, x, heads, offset)
+    want = ex.mlp(v, x, heads=heads)
+    ex.close()
+    np.testing.assert_array_equal(got, want)

@@ -176,10 +176,16 @@ struct ChainNet {
     // lane order).
     const float* part = nullptr;
     uint32_t dsteps = 0;
+    bool vec = false;  // launch_chain_rows: the input takes 16-byte loads
 };
 bool chain_fits(uint32_t in, uint32_t hidden, uint32_t layers);
 void launch_chain(int precision, const ChainNet& net, const void* X, uint32_t rows, float* out,
                   const ChainPass* plan, uint32_t npass, hipStream_t s);
+// The whole network over rows that all need the whole head, from a row-major
+// f32 input (converted as it is staged): passes of consecutive row blocks, as
+// even as `cus` compute units allow, up to CHAIN_PASS_BLOCKS blocks each.
+void launch_chain_rows(int precision, ChainNet net, const float* X, uint32_t rows, float* out, uint32_t cus,
+                       hipStream_t s);
 // The first layer's product over X's columns from k step net.dsteps on (the
 // columns that stay fixed while a wave is solved: seat and public features),
 // without bias, into part (the layout ChainNet::part describes), for every

@@ -1619,14 +1619,25 @@ __device__ __forceinline__ size_t part_tile(uint32_t rb, uint32_t fb, uint32_t h
 
 __device__ __forceinline__ uint32_t pack16(uint16_t lo, uint16_t hi) { return (uint32_t)lo | ((uint32_t)hi << 16); }
 
+// Modes: the whole net over a plan's passes; the whole net with the first
+// layer started from a precomputed partial product; the partial product alone;
+// the whole net over consecutive row blocks of a row-major f32 input.
+constexpr int CHAIN_FULL = 0, CHAIN_PART = 1, CHAIN_STATIC = 2, CHAIN_ROWS = 3;
+
+// The a-th 16-row block of the pass.
+template <int MODE>
+__device__ __forceinline__ uint32_t chain_block(const ChainPass* __restrict__ ps, uint32_t rb0, uint32_t a) {
+    return MODE == CHAIN_ROWS ? rb0 + a : ps->rb[a];
+}
+
 // The head over the pass's RB row blocks (LDS operand, K = hidden): rg row
 // groups of RBW blocks each (RBW = ceil(RB / rg); a group's blocks past RB are
 // computed from in-bounds LDS and not stored) by 8 / rg column groups; the
 // wavefront's column blocks are c, c + 8 / rg, ... in steps of CHAIN_NB of
 // them. Row-major f32 out.
-template <int PREC, int RB, int RBW>
+template <int PREC, int RB, int RBW, int MODE>
 __device__ __forceinline__ void chain_head(const ChainNet& net, uint32_t rows, float* __restrict__ out,
-                                           const ChainPass* __restrict__ ps, uint32_t nt, uint32_t rg,
+                                           const ChainPass* __restrict__ ps, uint32_t rb0, uint32_t nt, uint32_t rg,
                                            const uint16_t* lds, uint32_t lane, uint32_t wave) {
     const uint32_t q = lane >> 4, r = lane & 15, ksn = net.hidden >> 5;
     const uint32_t cg = CHAIN_WAVES / rg, g = wave / cg, c = wave % cg, a0 = g * RBW;
@@ -1652,7 +1663,7 @@ __device__ __forceinline__ void chain_head(const ChainNet& net, uint32_t rows, f
 #pragma unroll
             for (int a = 0; a < RBW; a++) {
                 if (a0 + a >= RB) break;
-                const uint32_t m = ps->rb[a0 + a] * 16 + rr;
+                const uint32_t m = chain_block<MODE>(ps, rb0, a0 + a) * 16 + rr;
                 if (m >= rows) continue;
                 float* o = out + (size_t)m * net.heads + n;
 #pragma unroll
@@ -1666,17 +1677,15 @@ __device__ __forceinline__ void chain_head(const ChainNet& net, uint32_t rows, f
 // One pass of the whole network over the pass's RB 16-row blocks (RB <= 8):
 // stage their input operand in LDS, run the trunk layers in place, write the
 // head.
-// Modes: the whole net; the whole net with the first layer started from a
-// precomputed partial product; the partial product alone.
-constexpr int CHAIN_FULL = 0, CHAIN_PART = 1, CHAIN_STATIC = 2;
 template <int PREC, int RB, int MODE>
-__device__ __forceinline__ void chain_pass(const ChainNet& net, const uint16_t* __restrict__ X, uint32_t rows,
-                                           float* __restrict__ out, const ChainPass* __restrict__ ps,
+__device__ __forceinline__ void chain_pass(const ChainNet& net, const void* __restrict__ Xv, uint32_t rows,
+                                           float* __restrict__ out, const ChainPass* __restrict__ ps, uint32_t rb0,
                                            uint16_t* lds, uint32_t lane, uint32_t wave) {
     const uint32_t q = lane >> 4, r = lane & 15;
     const uint32_t hblk = net.hidden >> 4, ksn = net.hidden >> 5;
     const uint32_t nb = hblk > wave ? (hblk - wave + CHAIN_WAVES - 1) / CHAIN_WAVES : 0;
-    const uint32_t nt = (min(ps->cols, net.heads) + 15) >> 4;  // head column blocks the pass needs
+    // head column blocks the pass needs
+    const uint32_t nt = ((MODE == CHAIN_ROWS ? net.heads : min(ps->cols, net.heads)) + 15) >> 4;
     // The first layer's k steps [s0, s0 + sn) of each row block (a contiguous
     // run of 1 KB steps in X), packed in LDS in pass order: all of them, the
     // first dsteps (partial start) or the rest (the static product).
@@ -1684,12 +1693,48 @@ __device__ __forceinline__ void chain_pass(const ChainNet& net, const uint16_t* 
     constexpr bool part = MODE == CHAIN_PART;
     const uint32_t s0 = MODE == CHAIN_STATIC ? net.dsteps : 0;
     const uint32_t sn = MODE == CHAIN_STATIC ? ks0 - net.dsteps : part ? net.dsteps : ks0;
-    const uint32_t per = sn * 64;  // uint4 per row block
+    if constexpr (MODE == CHAIN_ROWS) {
+        // One wavefront converts one (block, step) at a time: lane l reads 8
+        // floats of row l % 16, so the step's 16 rows arrive as whole 128-byte
+        // lines and its 64 fragments leave as one contiguous KB. Rows past the
+        // last repeat it (their outputs are not stored).
+        const float* X = (const float*)Xv;
+#pragma unroll 4
+        for (uint32_t i = wave; i < RB * ks0; i += CHAIN_WAVES) {
+            const uint32_t a = i / ks0, s = i % ks0, m = min((rb0 + a) * 16 + r, rows - 1);
+            const float* src = X + (size_t)m * net.in + 32 * s + 8 * q;
+            float v[8];
+            if (net.vec) {
+                const float4v lo = *(const float4v*)src, hi = *(const float4v*)(src + 4);
 #pragma unroll
-    for (int a = 0; a < RB; a++) {
-        const uint4* src = (const uint4*)(X + ((size_t)ps->rb[a] * ks0 + s0) * 512);
-        uint4* dst = (uint4*)lds + a * per;
-        for (uint32_t i = threadIdx.x; i < per; i += CHAIN_WAVES * 64) dst[i] = src[i];
+                for (int k = 0; k < 4; k++) {
+                    v[k] = lo[k];
+                    v[4 + k] = hi[k];
+                }
+            } else {
+#pragma unroll
+                for (int k = 0; k < 8; k++) v[k] = src[k];
+            }
+            uint4 f;
+            auto two = [&](int k) {
+                return PREC == WC_F16 ? pack16(f32_to_f16_rn(v[k]), f32_to_f16_rn(v[k + 1]))
+                                      : pack16(f32_to_bf16_rn(v[k]), f32_to_bf16_rn(v[k + 1]));
+            };
+            f.x = two(0);
+            f.y = two(2);
+            f.z = two(4);
+            f.w = two(6);
+            ((uint4*)lds)[(size_t)i * 64 + lane] = f;
+        }
+    } else {
+        const uint16_t* X = (const uint16_t*)Xv;
+        const uint32_t per = sn * 64;  // uint4 per row block
+#pragma unroll
+        for (int a = 0; a < RB; a++) {
+            const uint4* src = (const uint4*)(X + ((size_t)ps->rb[a] * ks0 + s0) * 512);
+            uint4* dst = (uint4*)lds + a * per;
+            for (uint32_t i = threadIdx.x; i < per; i += CHAIN_WAVES * 64) dst[i] = src[i];
+        }
     }
     float4v acc[8][CHAIN_NB];
     if constexpr (part) {  // the first layer starts from the precomputed product of its other columns
@@ -1758,31 +1803,33 @@ __device__ __forceinline__ void chain_pass(const ChainNet& net, const uint16_t* 
     // row groups of RB / rg blocks, 8 / rg blocks per column step), so that
     // every wavefront has work and reads fewer operand fragments per product.
     if (nt <= 6 && RB >= 4)
-        chain_head<PREC, RB, (RB + 3) / 4>(net, rows, out, ps, nt, 4, lds, lane, wave);
+        chain_head<PREC, RB, (RB + 3) / 4, MODE>(net, rows, out, ps, rb0, nt, 4, lds, lane, wave);
     else if (nt <= 12 && RB >= 2)
-        chain_head<PREC, RB, (RB + 1) / 2>(net, rows, out, ps, nt, 2, lds, lane, wave);
+        chain_head<PREC, RB, (RB + 1) / 2, MODE>(net, rows, out, ps, rb0, nt, 2, lds, lane, wave);
     else
-        chain_head<PREC, RB, RB>(net, rows, out, ps, nt, 1, lds, lane, wave);
+        chain_head<PREC, RB, RB, MODE>(net, rows, out, ps, rb0, nt, 1, lds, lane, wave);
 }
 
-// One workgroup per pass of the plan (plan_chain orders the passes so that
-// the costly ones start first).
+// One workgroup per pass: of the plan (plan_chain orders the passes so that
+// the costly ones start first), or of `per` consecutive row blocks.
 template <int PREC, int MODE>
 __global__ __launch_bounds__(CHAIN_WAVES * 64) __attribute__((amdgpu_waves_per_eu(CHAIN_WAVES / 4, CHAIN_WAVES / 4))) void k_chain(
-    ChainNet net, const uint16_t* __restrict__ X, uint32_t rows, float* __restrict__ out,
-    const ChainPass* __restrict__ plan) {
+    ChainNet net, const void* __restrict__ X, uint32_t rows, float* __restrict__ out,
+    const ChainPass* __restrict__ plan, uint32_t per) {
     __shared__ __attribute__((aligned(16))) uint16_t lds[CHAIN_LDS_HALVES];
     const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const ChainPass* ps = plan + blockIdx.x;
-    switch (min(CHAIN_PASS_BLOCKS, ps->n)) {
-        case 8: chain_pass<PREC, 8, MODE>(net, X, rows, out, ps, lds, lane, wave); break;
-        case 7: chain_pass<PREC, 7, MODE>(net, X, rows, out, ps, lds, lane, wave); break;
-        case 6: chain_pass<PREC, 6, MODE>(net, X, rows, out, ps, lds, lane, wave); break;
-        case 5: chain_pass<PREC, 5, MODE>(net, X, rows, out, ps, lds, lane, wave); break;
-        case 4: chain_pass<PREC, 4, MODE>(net, X, rows, out, ps, lds, lane, wave); break;
-        case 3: chain_pass<PREC, 3, MODE>(net, X, rows, out, ps, lds, lane, wave); break;
-        case 2: chain_pass<PREC, 2, MODE>(net, X, rows, out, ps, lds, lane, wave); break;
-        case 1: chain_pass<PREC, 1, MODE>(net, X, rows, out, ps, lds, lane, wave); break;
+    const uint32_t rb0 = blockIdx.x * per;
+    const uint32_t n = MODE == CHAIN_ROWS ? min(per, ((rows + 15) >> 4) - rb0) : ps->n;
+    switch (min(CHAIN_PASS_BLOCKS, n)) {
+        case 8: chain_pass<PREC, 8, MODE>(net, X, rows, out, ps, rb0, lds, lane, wave); break;
+        case 7: chain_pass<PREC, 7, MODE>(net, X, rows, out, ps, rb0, lds, lane, wave); break;
+        case 6: chain_pass<PREC, 6, MODE>(net, X, rows, out, ps, rb0, lds, lane, wave); break;
+        case 5: chain_pass<PREC, 5, MODE>(net, X, rows, out, ps, rb0, lds, lane, wave); break;
+        case 4: chain_pass<PREC, 4, MODE>(net, X, rows, out, ps, rb0, lds, lane, wave); break;
+        case 3: chain_pass<PREC, 3, MODE>(net, X, rows, out, ps, rb0, lds, lane, wave); break;
+        case 2: chain_pass<PREC, 2, MODE>(net, X, rows, out, ps, rb0, lds, lane, wave); break;
+        case 1: chain_pass<PREC, 1, MODE>(net, X, rows, out, ps, rb0, lds, lane, wave); break;
         default: break;
     }
 }
@@ -1791,17 +1838,17 @@ void launch_chain(int precision, const ChainNet& net, const void* X, uint32_t ro
                   const ChainPass* plan, uint32_t npass, hipStream_t s) {
     if (rows == 0 || npass == 0) return;
     dim3 grid(npass), block(CHAIN_WAVES * 64);
-    const uint16_t* x = (const uint16_t*)X;
+    const void* x = X;
     if (precision == WC_F16) {
         if (net.part)
-            hipLaunchKernelGGL((k_chain<WC_F16, CHAIN_PART>), grid, block, 0, s, net, x, rows, out, plan);
+            hipLaunchKernelGGL((k_chain<WC_F16, CHAIN_PART>), grid, block, 0, s, net, x, rows, out, plan, 0u);
         else
-            hipLaunchKernelGGL((k_chain<WC_F16, CHAIN_FULL>), grid, block, 0, s, net, x, rows, out, plan);
+            hipLaunchKernelGGL((k_chain<WC_F16, CHAIN_FULL>), grid, block, 0, s, net, x, rows, out, plan, 0u);
     } else {
         if (net.part)
-            hipLaunchKernelGGL((k_chain<WC_BF16, CHAIN_PART>), grid, block, 0, s, net, x, rows, out, plan);
+            hipLaunchKernelGGL((k_chain<WC_BF16, CHAIN_PART>), grid, block, 0, s, net, x, rows, out, plan, 0u);
         else
-            hipLaunchKernelGGL((k_chain<WC_BF16, CHAIN_FULL>), grid, block, 0, s, net, x, rows, out, plan);
+            hipLaunchKernelGGL((k_chain<WC_BF16, CHAIN_FULL>), grid, block, 0, s, net, x, rows, out, plan, 0u);
     }
 }
 
@@ -1810,11 +1857,26 @@ void launch_chain_static(int precision, const ChainNet& net, const void* X, floa
     if (npass == 0) return;
     dim3 grid(npass), block(CHAIN_WAVES * 64);
     if (precision == WC_F16)
-        hipLaunchKernelGGL((k_chain<WC_F16, CHAIN_STATIC>), grid, block, 0, s, net, (const uint16_t*)X, 0u, part,
-                           plan);
+        hipLaunchKernelGGL((k_chain<WC_F16, CHAIN_STATIC>), grid, block, 0, s, net, X, 0u, part,
+                           plan, 0u);
     else
-        hipLaunchKernelGGL((k_chain<WC_BF16, CHAIN_STATIC>), grid, block, 0, s, net, (const uint16_t*)X, 0u, part,
-                           plan);
+        hipLaunchKernelGGL((k_chain<WC_BF16, CHAIN_STATIC>), grid, block, 0, s, net, X, 0u, part,
+                           plan, 0u);
+}
+
+void launch_chain_rows(int precision, ChainNet net, const float* X, uint32_t rows, float* out, uint32_t cus,
+                       hipStream_t s) {
+    if (rows == 0) return;
+    net.vec = (uintptr_t)X % 16 == 0;
+    const uint32_t nrb = (rows + 15) / 16, rounds = (nrb + CHAIN_PASS_BLOCKS * cus - 1) / (CHAIN_PASS_BLOCKS * cus);
+    const uint32_t per = (nrb + rounds * cus - 1) / (rounds * cus);
+    dim3 grid((nrb + per - 1) / per), block(CHAIN_WAVES * 64);
+    if (precision == WC_F16)
+        hipLaunchKernelGGL((k_chain<WC_F16, CHAIN_ROWS>), grid, block, 0, s, net, (const void*)X, rows, out,
+                           (const ChainPass*)nullptr, per);
+    else
+        hipLaunchKernelGGL((k_chain<WC_BF16, CHAIN_ROWS>), grid, block, 0, s, net, (const void*)X, rows, out,
+                           (const ChainPass*)nullptr, per);
 }
 
 }  // namespace wc

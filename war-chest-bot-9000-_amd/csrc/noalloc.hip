@@ -30,21 +30,6 @@ void* g_scratch[MAX_DEVICES] = {};  // the array's device address on each device
 
 size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
 
-// Passes of up to CHAIN_PASS_BLOCKS consecutive 16-row blocks, every pass
-// computing all `cols` head columns: the plan of rows that all need the
-// whole head, written on the device (no host buffer, no copy).
-__global__ void k_plan_consecutive(ChainPass* plan, uint32_t nrb, uint32_t cols) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    const uint32_t npass = (nrb + CHAIN_PASS_BLOCKS - 1) / CHAIN_PASS_BLOCKS;
-    if (i >= npass) return;
-    ChainPass ps;
-    ps.n = min(CHAIN_PASS_BLOCKS, nrb - i * CHAIN_PASS_BLOCKS);
-    for (uint32_t j = 0; j < CHAIN_PASS_BLOCKS; j++) ps.rb[j] = j < ps.n ? i * CHAIN_PASS_BLOCKS + j : 0u;
-    ps.cols = cols;
-    ps.pad[0] = ps.pad[1] = 0;
-    plan[i] = ps;
-}
-
 }  // namespace
 
 // The scratch array's address on `device`, looked up the first time a device
@@ -82,9 +67,11 @@ bool Executor::mlp_forward_noalloc(uint64_t version, uint32_t rows, const float*
         return false;
     }
     if (rows == 0) return true;
-    // The pieces of one call, 256-byte aligned: the pass plan (fused net), the
-    // 16-bit input operand (rows padded to GEMM_ROWS; compensated f16: hi and
-    // lo planes), the hidden activations (layer-by-layer nets).
+    // The pieces of one call, 256-byte aligned: the 16-bit input operand (rows
+    // padded to GEMM_ROWS; compensated f16: hi and lo planes) and the hidden
+    // activations of the layer-by-layer nets. The fused net needs no scratch,
+    // but keeps the bound its callers size their batches by: its operand and
+    // 48 bytes per 128 rows.
     const bool fused = (precision_ == WC_F16 || precision_ == WC_BF16) && chain_fits(ns.in, ns.hidden, ns.layers);
     const size_t esz = precision_ == WC_F16X ? 4 : 2;
     const size_t prow = precision_ == WC_PRECISE ? rows : gemm_rows(rows);
@@ -95,7 +82,7 @@ bool Executor::mlp_forward_noalloc(uint64_t version, uint32_t rows, const float*
         at = a + bytes;
         return a;
     };
-    const size_t o_plan = fused ? take(size_t(npass) * sizeof(ChainPass)) : 0;
+    if (fused) take(size_t(npass) * sizeof(ChainPass));
     const size_t o_x = precision_ == WC_PRECISE ? 0 : take(prow * ns.in * esz);
     const size_t hbytes = prow * ns.hidden * (precision_ == WC_PRECISE ? 4 : esz);
     const size_t o_h0 = fused ? 0 : take(hbytes), o_h1 = fused ? 0 : take(hbytes);
@@ -123,24 +110,20 @@ bool Executor::mlp_forward_noalloc(uint64_t version, uint32_t rows, const float*
             k = ns.hidden;
         }
         launch_head_exact(in, ns.hidden, (const float*)bank->Whead, bank->bhead, ns.heads, out, rows, s);
+    } else if (fused) {
+        launch_chain_rows(precision_, chain_net(*bank), x, rows, out, cus_, s);
     } else {
         void* xop = base + o_x;
         launch_to16(precision_, x, xop, rows, ns.in, false, s);
-        if (fused) {
-            ChainPass* plan = (ChainPass*)(base + o_plan);
-            hipLaunchKernelGGL(k_plan_consecutive, dim3((npass + 63) / 64), dim3(64), 0, s, plan, nrb, ns.heads);
-            launch_chain(precision_, chain_net(*bank), xop, rows, out, plan, npass, s);
-        } else {
-            const void* in = xop;
-            uint32_t k = ns.in;
-            for (uint32_t l = 0; l < ns.layers; l++) {
-                void* o = base + (l & 1 ? o_h1 : o_h0);
-                launch_gemm16(precision_, in, k, bank->W[l], bank->B[l], ns.hidden, o, rows, true, true, s);
-                in = o;
-                k = ns.hidden;
-            }
-            launch_gemm16(precision_, in, ns.hidden, bank->Whead, bank->bhead, ns.heads, out, rows, false, false, s);
+        const void* in = xop;
+        uint32_t k = ns.in;
+        for (uint32_t l = 0; l < ns.layers; l++) {
+            void* o = base + (l & 1 ? o_h1 : o_h0);
+            launch_gemm16(precision_, in, k, bank->W[l], bank->B[l], ns.hidden, o, rows, true, true, s);
+            in = o;
+            k = ns.hidden;
         }
+        launch_gemm16(precision_, in, ns.hidden, bank->Whead, bank->bhead, ns.heads, out, rows, false, false, s);
     }
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) {
