@@ -1637,15 +1637,15 @@ __device__ __forceinline__ uint32_t chain_block(const ChainPass* __restrict__ ps
 // them. Row-major f32 out.
 template <int PREC, int RB, int RBW, int MODE>
 __device__ __forceinline__ void chain_head(const ChainNet& net, uint32_t rows, float* __restrict__ out,
-                                           const ChainPass* __restrict__ ps, uint32_t rb0, uint32_t nt, uint32_t rg,
-                                           const uint16_t* lds, uint32_t lane, uint32_t wave) {
+                                           const ChainPass* __restrict__ ps, uint32_t rb0, uint32_t t0,
+                                           uint32_t nt, uint32_t rg, const uint16_t* lds, uint32_t lane, uint32_t wave) {
     const uint32_t q = lane >> 4, r = lane & 15, ksn = net.hidden >> 5;
     const uint32_t cg = CHAIN_WAVES / rg, g = wave / cg, c = wave % cg, a0 = g * RBW;
     const uint16_t* wh = net.w[net.layers];
     const float* bh = net.b[net.layers];
     const uint16_t* xs = lds + (size_t)a0 * ksn * 512;
     float4v acc[8][CHAIN_NB];
-    for (uint32_t c0 = 0; c0 < nt; c0 += cg * CHAIN_NB) {
+    for (uint32_t c0 = t0; c0 < nt; c0 += cg * CHAIN_NB) {
         const uint32_t end = min(nt, c0 + cg * CHAIN_NB);
         const uint32_t hb = end > c0 + c ? (end - c0 - c + cg - 1) / cg : 0;
         chain_blocks<PREC, RBW>(acc, hb, xs, ksn, wh, c0 + c, cg, lane);
@@ -1684,8 +1684,11 @@ __device__ __forceinline__ void chain_pass(const ChainNet& net, const void* __re
     const uint32_t q = lane >> 4, r = lane & 15;
     const uint32_t hblk = net.hidden >> 4, ksn = net.hidden >> 5;
     const uint32_t nb = hblk > wave ? (hblk - wave + CHAIN_WAVES - 1) / CHAIN_WAVES : 0;
-    // head column blocks the pass needs
-    const uint32_t nt = ((MODE == CHAIN_ROWS ? net.heads : min(ps->cols, net.heads)) + 15) >> 4;
+    // head column blocks the pass needs: all of them, or (consecutive rows) the
+    // blockIdx.y-th of gridDim.y shares
+    const uint32_t nta = ((MODE == CHAIN_ROWS ? net.heads : min(ps->cols, net.heads)) + 15) >> 4;
+    const uint32_t t0 = MODE == CHAIN_ROWS ? nta * blockIdx.y / gridDim.y : 0;
+    const uint32_t nt = MODE == CHAIN_ROWS ? nta * (blockIdx.y + 1) / gridDim.y : nta;
     // The first layer's k steps [s0, s0 + sn) of each row block (a contiguous
     // run of 1 KB steps in X), packed in LDS in pass order: all of them, the
     // first dsteps (partial start) or the rest (the static product).
@@ -1802,12 +1805,12 @@ __device__ __forceinline__ void chain_pass(const ChainNet& net, const void* __re
     // Head: the columns the pass's rows need, nt 16-column blocks. Few blocks go to groups of wavefronts that split the rows (rg
     // row groups of RB / rg blocks, 8 / rg blocks per column step), so that
     // every wavefront has work and reads fewer operand fragments per product.
-    if (nt <= 6 && RB >= 4)
-        chain_head<PREC, RB, (RB + 3) / 4, MODE>(net, rows, out, ps, rb0, nt, 4, lds, lane, wave);
-    else if (nt <= 12 && RB >= 2)
-        chain_head<PREC, RB, (RB + 1) / 2, MODE>(net, rows, out, ps, rb0, nt, 2, lds, lane, wave);
+    if (nt - t0 <= 6 && RB >= 4)
+        chain_head<PREC, RB, (RB + 3) / 4, MODE>(net, rows, out, ps, rb0, t0, nt, 4, lds, lane, wave);
+    else if (nt - t0 <= 12 && RB >= 2)
+        chain_head<PREC, RB, (RB + 1) / 2, MODE>(net, rows, out, ps, rb0, t0, nt, 2, lds, lane, wave);
     else
-        chain_head<PREC, RB, RB, MODE>(net, rows, out, ps, rb0, nt, 1, lds, lane, wave);
+        chain_head<PREC, RB, RB, MODE>(net, rows, out, ps, rb0, t0, nt, 1, lds, lane, wave);
 }
 
 // One workgroup per pass: of the plan (plan_chain orders the passes so that
@@ -1870,7 +1873,12 @@ void launch_chain_rows(int precision, ChainNet net, const float* X, uint32_t row
     net.vec = (uintptr_t)X % 16 == 0;
     const uint32_t nrb = (rows + 15) / 16, rounds = (nrb + CHAIN_PASS_BLOCKS * cus - 1) / (CHAIN_PASS_BLOCKS * cus);
     const uint32_t per = (nrb + rounds * cus - 1) / (rounds * cus);
-    dim3 grid((nrb + per - 1) / per), block(CHAIN_WAVES * 64);
+    // Few rows: idle CUs repeat the trunk to take a share of the head columns
+    // each, down to one 16-column block per wavefront (250 rows, 567 heads:
+    // 15.5 us against 21.2 us with one share).
+    const uint32_t passes = (nrb + per - 1) / per, blocks = (net.heads + 15) / 16;
+    const uint32_t shares = std::max(1u, std::min((blocks + CHAIN_WAVES - 1) / CHAIN_WAVES, cus / passes));
+    dim3 grid(passes, shares), block(CHAIN_WAVES * 64);
     if (precision == WC_F16)
         hipLaunchKernelGGL((k_chain<WC_F16, CHAIN_ROWS>), grid, block, 0, s, net, (const void*)X, rows, out,
                            (const ChainPass*)nullptr, per);
