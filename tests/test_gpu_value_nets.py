@@ -84,3 +84,28 @@ def test_fused_net_from_rows_equals_the_planned_passes(precision, inputs, hidden
     want = ex.mlp(v, x, heads=heads)
     ex.close()
     np.testing.assert_array_equal(got, want)
+
+
+# one to four row blocks per pass, two rounds of passes, widths that leave wavefronts idle
+@pytest.mark.parametrize("inputs,hidden,layers,heads,rows,offset", [
+    (512, 384, 3, 567, 1, 0), (32, 32, 1, 1, 17, 1), (160, 352, 8, 130, 250, 3), (512, 384, 3, 22, 5100, 0),
+    (96, 128, 2, 140, 16000, 2), (64, 64, 1, 33, 26000, 0)])
+def test_compensated_fused_net(inputs, hidden, layers, heads, rows, offset):
+    """From rows and from planned passes alike, and within the compensated operands' rounding of float64: each
+    layer's pairs hold 22 bits (2^-22 of the operand), its float32 sum of K terms rounds by at most K 2^-24 of
+    the sum of magnitudes; 1e-5 of the largest value covers eight such layers of up to 512 terms."""
+    say(f"case compensated fused net: {rows} rows, {inputs} -> {layers}x{hidden} -> {heads}, buffers + {offset} floats")
+    net = ww.synth_weights(ww.mlp_dims(inputs, hidden, layers, heads, pool=8), seed=rows)
+    x = ww.synth_features(rows, inputs, seed=rows + 1)
+    ex = ww.Executor(0, ww.WC_F16X)
+    v = ex.publish(net)
+    got = forward_on_device(ex, v, x, heads, offset)
+    want = ex.mlp(v, x, heads=heads)
+    ex.close()
+    np.testing.assert_array_equal(got, want)
+    h, at, k = x[:500].astype(np.float64), 0, inputs
+    for layer in range(layers):
+        w = net.w[at:at + k * hidden].reshape(k, hidden).astype(np.float64)
+        h, at, k = np.maximum(h @ w + net.b[layer * hidden:(layer + 1) * hidden], 0.0), at + k * hidden, hidden
+    ref = h @ net.w[at:].reshape(heads, hidden).T.astype(np.float64) + net.b[layers * hidden:]
+    assert np.abs(got[:500] - ref).max() <= 1e-5 * np.abs(ref).max()

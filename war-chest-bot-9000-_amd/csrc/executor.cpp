@@ -478,7 +478,8 @@ bool Executor::upload(const WaveHost& w, const NetBank& bank, uint32_t slot, std
     o.head_tile_n = blob.put(w.head_tile_n);
     std::vector<ChainPass> plan[2];
     for (int p = 0; p < 2; p++) {
-        plan[p] = plan_chain(w.head_rb_n[p].data(), (uint32_t)w.head_rb_n[p].size(), w.net.heads, cus_);
+        plan[p] = plan_chain(w.head_rb_n[p].data(), (uint32_t)w.head_rb_n[p].size(), w.net.heads, cus_,
+                             chain_most(precision_));
         if (!check_chain_plan(plan[p], w.head_rb_n[p].data(), (uint32_t)w.head_rb_n[p].size(), w.net.heads, err))
             return false;
         o.hb[p] = blob.put(w.head_rb_n[p]);
@@ -758,8 +759,9 @@ void Executor::run_mlp(const NetBank& bank, uint32_t rows, const void* x, std::v
             marks->push_back(e);
         }
     };
-    if ((precision_ == WC_F16 || precision_ == WC_BF16) && chain_fits(ns.in, ns.hidden, ns.layers)) {
+    if (precision_ != WC_PRECISE && chain_fits(ns.in, ns.hidden, ns.layers)) {
         ChainNet net = chain_net(bank);
+        net.xplane = size_t(gemm_rows(rows)) * ns.in;
         if (part) {
             net.part = part;
             net.dsteps = 2 * ns.pool / 32;
@@ -1466,7 +1468,7 @@ bool Executor::mlp_forward(uint64_t version, uint32_t rows, const float* x, floa
         return a;
     };
     const size_t prow = precision_ == WC_PRECISE ? rows : gemm_rows(rows);  // GEMM operands: padded rows
-    const std::vector<ChainPass> plan = plan_chain(nullptr, (rows + 15) / 16, ns.heads, cus_);
+    const std::vector<ChainPass> plan = plan_chain(nullptr, (rows + 15) / 16, ns.heads, cus_, chain_most(precision_));
     if (!check_chain_plan(plan, nullptr, (rows + 15) / 16, ns.heads, err)) return false;
     size_t m_x = mtake(prow * ns.in * esz), m_h0 = mtake(prow * ns.hidden * esz), m_h1 = mtake(prow * ns.hidden * esz),
            m_out = mtake(size_t(rows) * ns.heads * 4), m_stage = mtake(size_t(rows) * ns.in * 4),

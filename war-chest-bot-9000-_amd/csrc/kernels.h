@@ -156,7 +156,7 @@ void launch_head_exact(const float* H, uint32_t hidden, const float* Wh, const f
 void launch_gemm16(int precision, const void* X, uint32_t K, const void* Wt, const float* b, uint32_t N,
                    void* Y, uint32_t M, bool relu, bool out16, hipStream_t s, const uint32_t* tile_n = nullptr);
 // Whole-network MLP in one launch (16-bit operands, f32 accumulate): one
-// workgroup per pass of a plan (plan_chain), each running its up to 128 rows
+// workgroup per pass of a plan (plan_chain, chain_most), each running its up to 128 rows
 // through every layer with the activations resident in LDS; writes out[r, k]
 // (row-major f32, `heads` columns) for r < rows and the columns k < the pass's
 // cols. X is the fragment-major input with gemm_rows(rows) rows; w/b hold the
@@ -176,14 +176,17 @@ struct ChainNet {
     // lane order).
     const float* part = nullptr;
     uint32_t dsteps = 0;
+    size_t xplane = 0;  // compensated f16: elements between the input's hi and lo planes
     bool vec = false;  // launch_chain_rows: the input takes 16-byte loads
 };
+// Blocks a pass holds: a compensated operand takes twice the LDS.
+uint32_t chain_most(int precision);
 bool chain_fits(uint32_t in, uint32_t hidden, uint32_t layers);
 void launch_chain(int precision, const ChainNet& net, const void* X, uint32_t rows, float* out,
                   const ChainPass* plan, uint32_t npass, hipStream_t s);
 // The whole network over rows that all need the whole head, from a row-major
 // f32 input (converted as it is staged): passes of consecutive row blocks, as
-// even as `cus` compute units allow, up to CHAIN_PASS_BLOCKS blocks each.
+// even as `cus` compute units allow, up to chain_most blocks each.
 void launch_chain_rows(int precision, ChainNet net, const float* X, uint32_t rows, float* out, uint32_t cus,
                        hipStream_t s);
 // The first layer's product over X's columns from k step net.dsteps on (the

@@ -1513,6 +1513,8 @@ bool chain_fits(uint32_t in, uint32_t hidden, uint32_t layers) {
            hidden <= CHAIN_WAVES * CHAIN_NB * 16 && layers >= 1 && layers <= CHAIN_MAX_LAYERS;
 }
 
+uint32_t chain_most(int precision) { return precision == WC_F16X ? CHAIN_PASS_BLOCKS / 2 : CHAIN_PASS_BLOCKS; }
+
 template <int PREC>
 __device__ __forceinline__ float4v mfma16(const uint4& a, const uint4& b, const float4v& c) {
     if (PREC == WC_F16)
@@ -1837,12 +1839,247 @@ __global__ __launch_bounds__(CHAIN_WAVES * 64) __attribute__((amdgpu_waves_per_e
     }
 }
 
+// ------------------------------------- fused leaf network, compensated f16
+//
+// k_chain for operands held as f16 pairs hi + lo: both planes of up to four
+// row blocks live in LDS, and each step's product is lo hi + hi lo + hi hi, as
+// k_gemm_x takes it (x's lo first). Products, order and rounding are
+// k_gemm_x's, so the results are too, bit for bit.
+//
+// Bound: a pass streams both planes of every weight matrix from L2 (2.8 MB
+// for the 512 -> 3x384 -> 567 net, at 64 bytes per clock and CU) under three
+// MFMAs per tile and step, against one read and write of every activation
+// plane through HBM per layer and 93 workgroups for 3,915 rows in k_gemm_x. In
+// the 64-subgame wave a pass (3,915 rows, head widths per block) takes 38 us
+// against 133; 5,003 rows with 22 heads take 30 us against 132.
+
+constexpr int CHAINX_RB = 4;
+
+template <int NB, int RB>
+__device__ __forceinline__ void chainx_kloop(float4v (&acc)[CHAINX_RB][CHAIN_NB], const uint16_t* xs, uint32_t xplane,
+                                             uint32_t ks, const uint16_t* __restrict__ wp, size_t wstride,
+                                             size_t wplane) {
+#pragma unroll
+    for (int a = 0; a < RB; a++)
+#pragma unroll
+        for (int b = 0; b < NB; b++) acc[a][b] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
+    uint4 xa[2][RB], xb[2][RB], w0[2][NB], w1[2][NB], w2[2][NB], w3[2][NB];
+    auto ldw = [&](uint4 (&fw)[2][NB], uint32_t s) {
+        s = s < ks ? s : ks - 1;
+#pragma unroll
+        for (int b = 0; b < NB; b++) {
+            const uint16_t* p = wp + b * wstride + (size_t)s * 512;
+            fw[0][b] = *(const uint4*)p;
+            fw[1][b] = *(const uint4*)(p + wplane);
+        }
+    };
+    auto ldx = [&](uint4 (&fx)[2][RB], uint32_t s) {
+        s = s < ks ? s : ks - 1;
+#pragma unroll
+        for (int a = 0; a < RB; a++) {
+            const uint16_t* p = xs + ((size_t)a * ks + s) * 512;
+            fx[0][a] = *(const uint4*)p;
+            fx[1][a] = *(const uint4*)(p + xplane);
+        }
+    };
+    auto step = [&](const uint4 (&fx)[2][RB], const uint4 (&fw)[2][NB]) {
+#pragma unroll
+        for (int a = 0; a < RB; a++)
+#pragma unroll
+            for (int b = 0; b < NB; b++) acc[a][b] = mfma16<WC_F16>(fw[0][b], fx[1][a], acc[a][b]);
+#pragma unroll
+        for (int a = 0; a < RB; a++)
+#pragma unroll
+            for (int b = 0; b < NB; b++) acc[a][b] = mfma16<WC_F16>(fw[1][b], fx[0][a], acc[a][b]);
+#pragma unroll
+        for (int a = 0; a < RB; a++)
+#pragma unroll
+            for (int b = 0; b < NB; b++) acc[a][b] = mfma16<WC_F16>(fw[0][b], fx[0][a], acc[a][b]);
+    };
+    ldw(w0, 0);
+    ldw(w1, 1);
+    ldx(xa, 0);
+    uint32_t s = 0;
+    for (; s + 4 <= ks; s += 4) {
+        ldw(w2, s + 2);
+        ldx(xb, s + 1);
+        __builtin_amdgcn_sched_barrier(0);
+        step(xa, w0);
+        __builtin_amdgcn_sched_barrier(0);
+        ldw(w3, s + 3);
+        ldx(xa, s + 2);
+        __builtin_amdgcn_sched_barrier(0);
+        step(xb, w1);
+        __builtin_amdgcn_sched_barrier(0);
+        ldw(w0, s + 4);
+        ldx(xb, s + 3);
+        __builtin_amdgcn_sched_barrier(0);
+        step(xa, w2);
+        __builtin_amdgcn_sched_barrier(0);
+        ldw(w1, s + 5);
+        ldx(xa, s + 4);
+        __builtin_amdgcn_sched_barrier(0);
+        step(xb, w3);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    for (; s < ks; s++) {  // K not a multiple of 128: the last steps one at a time
+        ldw(w0, s);
+        ldx(xa, s);
+        step(xa, w0);
+    }
+}
+
+// The wavefront's column blocks blk0, blk0 + CHAIN_WAVES, ... (nb of them) of
+// a matrix with N columns.
+template <int RB>
+__device__ __forceinline__ void chainx_blocks(float4v (&acc)[CHAINX_RB][CHAIN_NB], uint32_t nb, const uint16_t* lds,
+                                              uint32_t xplane, uint32_t ks, const uint16_t* __restrict__ W,
+                                              uint32_t N, uint32_t blk0, uint32_t lane) {
+    const uint16_t* xs = lds + lane * 8;
+    const uint16_t* wp = W + ((size_t)blk0 * ks * 64 + lane) * 8;
+    const size_t wstride = (size_t)CHAIN_WAVES * ks * 512;
+    const size_t wplane = (size_t)((N + GEMM_ROWS - 1) / GEMM_ROWS * GEMM_ROWS) * ks * 32;
+    if (nb == 1)
+        chainx_kloop<1, RB>(acc, xs, xplane, ks, wp, wstride, wplane);
+    else if (nb == 2)
+        chainx_kloop<2, RB>(acc, xs, xplane, ks, wp, wstride, wplane);
+    else if (nb == 3)
+        chainx_kloop<3, RB>(acc, xs, xplane, ks, wp, wstride, wplane);
+}
+
+// An f16 pair of v: hi = f16(v), lo = f16(v - hi).
+__device__ __forceinline__ void split16(float v, uint16_t* hi, uint16_t* lo) {
+    *hi = f32_to_f16_rn(v);
+    *lo = f32_to_f16_rn(v - (float)__builtin_bit_cast(_Float16, *hi));
+}
+
+template <int RB, int MODE>
+__device__ __forceinline__ void chainx_pass(const ChainNet& net, const void* __restrict__ Xv, uint32_t rows,
+                                            float* __restrict__ out, const ChainPass* __restrict__ ps, uint32_t rb0,
+                                            uint16_t* lds, uint32_t lane, uint32_t wave) {
+    const uint32_t q = lane >> 4, r = lane & 15;
+    const uint32_t hblk = net.hidden >> 4, ksn = net.hidden >> 5, ks0 = net.in >> 5;
+    const uint32_t nb = hblk > wave ? (hblk - wave + CHAIN_WAVES - 1) / CHAIN_WAVES : 0;
+    const uint32_t nta = ((MODE == CHAIN_ROWS ? net.heads : min(ps->cols, net.heads)) + 15) >> 4;
+    const uint32_t t0 = MODE == CHAIN_ROWS ? nta * blockIdx.y / gridDim.y : 0;
+    const uint32_t nt = MODE == CHAIN_ROWS ? nta * (blockIdx.y + 1) / gridDim.y : nta;
+    const uint32_t plane = RB * max(ks0, ksn) * 512;  // halves between the planes in LDS
+    if constexpr (MODE == CHAIN_ROWS) {  // as chain_pass stages it, both planes
+        const float* X = (const float*)Xv;
+#pragma unroll 2
+        for (uint32_t i = wave; i < RB * ks0; i += CHAIN_WAVES) {
+            const uint32_t a = i / ks0, s = i % ks0, m = min((rb0 + a) * 16 + r, rows - 1);
+            const float* src = X + (size_t)m * net.in + 32 * s + 8 * q;
+            float v[8];
+            if (net.vec) {
+                const float4v lo = *(const float4v*)src, hi = *(const float4v*)(src + 4);
+#pragma unroll
+                for (int k = 0; k < 4; k++) {
+                    v[k] = lo[k];
+                    v[4 + k] = hi[k];
+                }
+            } else {
+#pragma unroll
+                for (int k = 0; k < 8; k++) v[k] = src[k];
+            }
+            uint16_t h[8], l[8];
+#pragma unroll
+            for (int k = 0; k < 8; k++) split16(v[k], h + k, l + k);
+            uint16_t* dst = lds + ((size_t)i * 64 + lane) * 8;
+            *(uint4*)dst = make_uint4(pack16(h[0], h[1]), pack16(h[2], h[3]), pack16(h[4], h[5]), pack16(h[6], h[7]));
+            *(uint4*)(dst + plane) =
+                make_uint4(pack16(l[0], l[1]), pack16(l[2], l[3]), pack16(l[4], l[5]), pack16(l[6], l[7]));
+        }
+    } else {
+        const uint16_t* X = (const uint16_t*)Xv;
+        const uint32_t per = ks0 * 64;  // uint4 per row block and plane
+#pragma unroll
+        for (int a = 0; a < RB; a++) {
+            const uint4* hi = (const uint4*)(X + (size_t)ps->rb[a] * ks0 * 512);
+            const uint4* lo = (const uint4*)(X + net.xplane + (size_t)ps->rb[a] * ks0 * 512);
+            uint4* dst = (uint4*)lds + a * per;
+            for (uint32_t i = threadIdx.x; i < per; i += CHAIN_WAVES * 64) {
+                dst[i] = hi[i];
+                *(uint4*)((uint16_t*)(dst + i) + plane) = lo[i];
+            }
+        }
+    }
+    float4v acc[CHAINX_RB][CHAIN_NB];
+    __syncthreads();
+    for (uint32_t l = 0; l < net.layers; l++) {
+        chainx_blocks<RB>(acc, nb, lds, plane, l ? ksn : ks0, net.w[l], net.hidden, wave, lane);
+        __syncthreads();  // the layer input is dead from here on
+        const float* bias = net.b[l];
+#pragma unroll
+        for (int b = 0; b < CHAIN_NB; b++) {
+            if ((uint32_t)b >= nb) break;
+            const uint32_t n = (wave + CHAIN_WAVES * b) * 16 + 4 * q;
+            float bv[4];
+#pragma unroll
+            for (int v = 0; v < 4; v++) bv[v] = bias[n + v];
+            const size_t col = (size_t)(n >> 5) * 64 + r + ((n & 31) >> 3) * 16;
+#pragma unroll
+            for (int a = 0; a < RB; a++) {
+                uint16_t h[4], lo[4];
+#pragma unroll
+                for (int v = 0; v < 4; v++) {
+                    const float y = acc[a][b][v] + bv[v];
+                    split16(y > 0.0f ? y : 0.0f, h + v, lo + v);
+                }
+                uint16_t* dst = lds + (((size_t)a * ksn * 64 + col) * 8 + (n & 7));
+                *(uint2*)dst = make_uint2(pack16(h[0], h[1]), pack16(h[2], h[3]));
+                *(uint2*)(dst + plane) = make_uint2(pack16(lo[0], lo[1]), pack16(lo[2], lo[3]));
+            }
+        }
+        __syncthreads();
+    }
+    const float* bh = net.b[net.layers];
+    for (uint32_t c0 = t0; c0 < nt; c0 += CHAIN_WAVES * CHAIN_NB) {
+        const uint32_t end = min(nt, c0 + CHAIN_WAVES * CHAIN_NB);
+        const uint32_t hb = end > c0 + wave ? (end - c0 - wave + CHAIN_WAVES - 1) / CHAIN_WAVES : 0;
+        chainx_blocks<RB>(acc, hb, lds, plane, ksn, net.w[net.layers], net.heads, c0 + wave, lane);
+#pragma unroll
+        for (int b = 0; b < CHAIN_NB; b++) {
+            if ((uint32_t)b >= hb) break;
+            const uint32_t n = (c0 + wave + CHAIN_WAVES * b) * 16 + 4 * q;
+#pragma unroll
+            for (int a = 0; a < RB; a++) {
+                const uint32_t m = chain_block<MODE>(ps, rb0, a) * 16 + r;
+                if (m >= rows) continue;
+#pragma unroll
+                for (int v = 0; v < 4; v++)
+                    if (n + v < net.heads) out[(size_t)m * net.heads + n + v] = acc[a][b][v] + bh[n + v];
+            }
+        }
+    }
+}
+
+template <int MODE>
+__global__ __launch_bounds__(CHAIN_WAVES * 64) __attribute__((amdgpu_waves_per_eu(CHAIN_WAVES / 4, CHAIN_WAVES / 4))) void k_chain_x(
+    ChainNet net, const void* __restrict__ X, uint32_t rows, float* __restrict__ out,
+    const ChainPass* __restrict__ plan, uint32_t per) {
+    __shared__ __attribute__((aligned(16))) uint16_t lds[CHAIN_LDS_HALVES];
+    const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const ChainPass* ps = plan + blockIdx.x;
+    const uint32_t rb0 = blockIdx.x * per;
+    const uint32_t n = MODE == CHAIN_ROWS ? min(per, ((rows + 15) >> 4) - rb0) : ps->n;
+    switch (min((uint32_t)CHAINX_RB, n)) {
+        case 4: chainx_pass<4, MODE>(net, X, rows, out, ps, rb0, lds, lane, wave); break;
+        case 3: chainx_pass<3, MODE>(net, X, rows, out, ps, rb0, lds, lane, wave); break;
+        case 2: chainx_pass<2, MODE>(net, X, rows, out, ps, rb0, lds, lane, wave); break;
+        case 1: chainx_pass<1, MODE>(net, X, rows, out, ps, rb0, lds, lane, wave); break;
+        default: break;
+    }
+}
+
 void launch_chain(int precision, const ChainNet& net, const void* X, uint32_t rows, float* out,
                   const ChainPass* plan, uint32_t npass, hipStream_t s) {
     if (rows == 0 || npass == 0) return;
     dim3 grid(npass), block(CHAIN_WAVES * 64);
     const void* x = X;
-    if (precision == WC_F16) {
+    if (precision == WC_F16X) {
+        hipLaunchKernelGGL(k_chain_x<CHAIN_FULL>, grid, block, 0, s, net, x, rows, out, plan, 0u);
+    } else if (precision == WC_F16) {
         if (net.part)
             hipLaunchKernelGGL((k_chain<WC_F16, CHAIN_PART>), grid, block, 0, s, net, x, rows, out, plan, 0u);
         else
@@ -1871,7 +2108,7 @@ void launch_chain_rows(int precision, ChainNet net, const float* X, uint32_t row
                        hipStream_t s) {
     if (rows == 0) return;
     net.vec = (uintptr_t)X % 16 == 0;
-    const uint32_t nrb = (rows + 15) / 16, rounds = (nrb + CHAIN_PASS_BLOCKS * cus - 1) / (CHAIN_PASS_BLOCKS * cus);
+    const uint32_t nrb = (rows + 15) / 16, most = chain_most(precision), rounds = (nrb + most * cus - 1) / (most * cus);
     const uint32_t per = (nrb + rounds * cus - 1) / (rounds * cus);
     // Few rows: idle CUs repeat the trunk to take a share of the head columns
     // each, down to one 16-column block per wavefront (250 rows, 567 heads:
@@ -1879,7 +2116,10 @@ void launch_chain_rows(int precision, ChainNet net, const float* X, uint32_t row
     const uint32_t passes = (nrb + per - 1) / per, blocks = (net.heads + 15) / 16;
     const uint32_t shares = std::max(1u, std::min((blocks + CHAIN_WAVES - 1) / CHAIN_WAVES, cus / passes));
     dim3 grid(passes, shares), block(CHAIN_WAVES * 64);
-    if (precision == WC_F16)
+    if (precision == WC_F16X)
+        hipLaunchKernelGGL(k_chain_x<CHAIN_ROWS>, grid, block, 0, s, net, (const void*)X, rows, out,
+                           (const ChainPass*)nullptr, per);
+    else if (precision == WC_F16)
         hipLaunchKernelGGL((k_chain<WC_F16, CHAIN_ROWS>), grid, block, 0, s, net, (const void*)X, rows, out,
                            (const ChainPass*)nullptr, per);
     else

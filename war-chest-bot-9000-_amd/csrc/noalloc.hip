@@ -71,8 +71,8 @@ bool Executor::mlp_forward_noalloc(uint64_t version, uint32_t rows, const float*
     // padded to GEMM_ROWS; compensated f16: hi and lo planes) and the hidden
     // activations of the layer-by-layer nets. The fused net needs no scratch,
     // but keeps the bound its callers size their batches by: its operand and
-    // 48 bytes per 128 rows.
-    const bool fused = (precision_ == WC_F16 || precision_ == WC_BF16) && chain_fits(ns.in, ns.hidden, ns.layers);
+    // 48 bytes per 128 rows, or (compensated f16) the layer-by-layer pieces.
+    const bool fused = precision_ != WC_PRECISE && chain_fits(ns.in, ns.hidden, ns.layers);
     const size_t esz = precision_ == WC_F16X ? 4 : 2;
     const size_t prow = precision_ == WC_PRECISE ? rows : gemm_rows(rows);
     const uint32_t nrb = (rows + 15) / 16, npass = (nrb + CHAIN_PASS_BLOCKS - 1) / CHAIN_PASS_BLOCKS;
@@ -82,10 +82,11 @@ bool Executor::mlp_forward_noalloc(uint64_t version, uint32_t rows, const float*
         at = a + bytes;
         return a;
     };
-    if (fused) take(size_t(npass) * sizeof(ChainPass));
+    if (fused && precision_ != WC_F16X) take(size_t(npass) * sizeof(ChainPass));
     const size_t o_x = precision_ == WC_PRECISE ? 0 : take(prow * ns.in * esz);
     const size_t hbytes = prow * ns.hidden * (precision_ == WC_PRECISE ? 4 : esz);
-    const size_t o_h0 = fused ? 0 : take(hbytes), o_h1 = fused ? 0 : take(hbytes);
+    const bool acts = !fused || precision_ == WC_F16X;
+    const size_t o_h0 = acts ? take(hbytes) : 0, o_h1 = acts ? take(hbytes) : 0;
     if (at > WC_NOALLOC_SCRATCH_BYTES) {
         const size_t per_row = std::max<size_t>(at / std::max<uint32_t>(rows, 1), 1);
         *err = std::to_string(rows) + " rows need " + std::to_string(at) + " bytes of scratch; the allocation-free "

@@ -2040,7 +2040,7 @@ bool check_chain_plan(const std::vector<ChainPass>& plan, const uint32_t* cols, 
     return true;
 }
 
-std::vector<ChainPass> plan_chain(const uint32_t* cols, uint32_t nrb, uint32_t heads, uint32_t cus) {
+std::vector<ChainPass> plan_chain(const uint32_t* cols, uint32_t nrb, uint32_t heads, uint32_t cus, uint32_t most) {
     std::vector<ChainPass> out;
     if (!nrb) return out;
     cus = std::max(cus, 1u);
@@ -2066,9 +2066,9 @@ std::vector<ChainPass> plan_chain(const uint32_t* cols, uint32_t nrb, uint32_t h
     // A pass also closes before its cost would exceed that of a full pass of
     // narrow (64-column) blocks, so passes of wide-head blocks hold fewer rows
     // and the longest passes, which start first, stay short.
-    const double cap = (pass_cost + CHAIN_PASS_BLOCKS * (1.0 + col_cost * 4)) * (1.0 + 1e-9);
+    const double cap = (pass_cost + most * (1.0 + col_cost * 4)) * (1.0 + 1e-9);
     auto closes = [&](uint32_t pn, double pc, uint32_t i) {
-        return pn == CHAIN_PASS_BLOCKS || (pn > 0 && pass_cost + pc + c[i] > cap);
+        return pn == most || (pn > 0 && pass_cost + pc + c[i] > cap);
     };
     // Shares of consecutive blocks under a cost bound t; returns their ends.
     auto deal = [&](double t, std::vector<uint32_t>* ends) {

@@ -145,8 +145,10 @@ static_assert(sizeof(ChainPass) == 12 * 4, "ChainPass is 48 bytes");
 // listed by estimated cost, longest first: run in list order on CUs that take
 // the next pass as they free up (longest-processing-time-first list
 // scheduling), the last passes end at about the same time. Every block is in
-// exactly one pass.
-std::vector<ChainPass> plan_chain(const uint32_t* cols, uint32_t nrb, uint32_t heads, uint32_t cus);
+// exactly one pass. `most` (at most CHAIN_PASS_BLOCKS) bounds the blocks of a
+// pass.
+std::vector<ChainPass> plan_chain(const uint32_t* cols, uint32_t nrb, uint32_t heads, uint32_t cus,
+                                  uint32_t most = CHAIN_PASS_BLOCKS);
 // What the fused kernel assumes of a plan: every block below nrb in exactly
 // one pass, 1..CHAIN_PASS_BLOCKS blocks per pass, and each pass's cols at
 // least every one of its blocks' widths.
