@@ -603,6 +603,7 @@ bool Executor::upload(const WaveHost& w, const NetBank& bank, uint32_t slot, std
         d.leaf_rec[p] = (const LeafRec*)(T + o.lr[p]);
         d.pool_grp[p] = (const PoolGroup*)(T + o.pg[p]);
         d.npool[p] = (uint32_t)w.pool_grp[p].size();
+        d.nlong[p] = pool_long_groups(w.pool_grp[p].data(), d.npool[p]);
         d.nleaf[p] = (uint32_t)w.leaf_rec[p].size();
         d.tower_blk[p] = (const TowerBlock*)(T + o.twb[p]);
         d.tower_unit[p] = (const TowerUnit*)(T + o.twu[p]);
@@ -630,6 +631,7 @@ bool Executor::upload(const WaveHost& w, const NetBank& bank, uint32_t slot, std
     d.max_rwin = w.max_rwin;
     d.unit_lds = unit_lds_ ? 1u : 0u;
     d.nsub = w.nsub;
+    d.emb_wide = uint64_t(ncfg) * ns.pool * 4 > UINT32_MAX ? 1u : 0u;
     d.regret = (float*)(A + a_regret);
     d.cur = (float*)(A + a_cur);
     d.sum = (float*)(A + a_sum);

@@ -58,8 +58,10 @@ struct WaveDev {
     uint32_t max_vwin;  // widest unit value window (floats)
     uint32_t max_rwin;  // widest unit reach window (floats)
     uint32_t unit_lds;  // 1: the sweep and reach passes keep unit windows in LDS when they fit
+    uint32_t emb_wide;  // 1: the embedding table's byte offsets need 64 bits
     uint32_t ndec[2];
     uint32_t npool[2];  // pool groups of each player
+    uint32_t nlong[2];  // of them, the leading ones that take a workgroup each (pool_long_groups)
     uint32_t nleaf[2];  // network-leaf slots of each player (leaf_rec entries)
     const TowerBlock* tower_blk[2];  // two-tower readout blocks and tiles of each player
     const TowerUnit* tower_unit[2];
@@ -112,6 +114,9 @@ void launch_seed_sum(const WaveDev& w, hipStream_t s);
 // discount and this iteration's addition, search.rs:1770-1779,1818-1835), in
 // workgroups of their own: it reads only the final reach and cur, as the
 // leaf input does.
+// The leading groups of a player's list (longest config lists first) that the
+// 16-bit pooling gives a workgroup each.
+uint32_t pool_long_groups(const PoolGroup* grp, uint32_t n);
 void launch_pool(const WaveDev& w, int player, int precision, void* x0, void* x1, hipStream_t s, int acc = -1,
                  float ds = 1.0f);
 // Seat and public features of both query inputs (once per upload).

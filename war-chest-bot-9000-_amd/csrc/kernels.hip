@@ -444,9 +444,15 @@ __device__ __forceinline__ float lane_sum_in_order(float tot, float v, uint32_t 
 // reach (normalize_weights, engine/src/rebel.rs:1054-1068; accumulate,
 // net.rs:161-170). Lanes load 64 configs at a time; both reductions then run
 // in config order with every lane holding the running value, so the result is
-// the CPU's sequential sum. The pooled block goes straight into the two query
-// inputs that carry it: [pooled_q | pooled_{1-q} | seat | public] for
+// the CPU's sequential sum. Bound: the instructions of the longest list's chain
+// (a lane per dimension, configs one after another), so each config costs a
+// lane read, a 32-bit add and a load for its embedding (64-bit addresses cost
+// five more scalar instructions) and a lane read, a product and a sum, with 16
+// configs' loads in flight ahead of them: 64 depth-1 subgames 52 -> 32 us per
+// launch, 32 depth-2 subgames 48 -> 30 us. WIDE: a table of 4 GiB or more.
+// The pooled block goes straight into the two query inputs that carry it: [pooled_q | pooled_{1-q} | seat | public] for
 // traverser q.
+template <bool WIDE>
 __global__ __launch_bounds__(BLOCK) void k_pool_exact(WaveDev w, int player, float* x0, float* x1, int acc,
                                                     float ds, uint32_t pool_blocks) {
     uint32_t pbk;
@@ -487,27 +493,55 @@ __global__ __launch_bounds__(BLOCK) void k_pool_exact(WaveDev w, int player, flo
         const uint32_t k = k0 + lane;
         const bool live = k < pool;
         float acc = 0.0f;
+        // 16 configs' embeddings per batch, one batch loading while the one
+        // before it is added in config order. Lanes past the list hold config
+        // 0, so that a batch's loads need no branch.
+        float e0[16], e1[16];
+        const uint32_t kk = live ? k : 0u;
+        auto index = [&](uint32_t c0) { return (c0 + lane < n ? cfgs[c0 + lane] : 0u) * (WIDE ? 1u : pool); };
+        auto belief = [&](uint32_t c0) { return c0 + lane < n ? r[c0 + lane] * scale + flat : 0.0f; };
+        auto fetch = [&](float (&e)[16], uint32_t cf, uint32_t j0) {
+#pragma unroll
+            for (uint32_t j = 0; j < 16; j++) {
+                const uint32_t c = lane_value(cf, j0 + j);
+                if (WIDE)
+                    e[j] = w.cfg_emb[(size_t)c * pool + kk];
+                else  // a 32-bit byte offset from the table
+                    e[j] = *(const float*)((const char*)w.cfg_emb + 4u * (c + kk));
+            }
+        };
+        auto add = [&](const float (&e)[16], float beta, uint32_t j0, uint32_t left) {
+            if (left >= 16) {
+#pragma unroll
+                for (uint32_t j = 0; j < 16; j++) acc += lane_value(beta, j0 + j) * e[j];
+                return;
+            }
+#pragma unroll
+            for (uint32_t j = 0; j < 16; j++)
+                if (j < left) acc += lane_value(beta, j0 + j) * e[j];
+        };
+        uint32_t cf = index(0);
+        float beta = belief(0);
+        fetch(e0, cf, 0);
         for (uint32_t c0 = 0; c0 < n; c0 += 64) {
-            uint32_t cf = c0 + lane < n ? cfgs[c0 + lane] : 0u;
-            float beta = c0 + lane < n ? r[c0 + lane] * scale + flat : 0.0f;
-            uint32_t m = n - c0 < 64 ? n - c0 : 64;
-            uint32_t j = 0;
-            for (; j + 8 <= m; j += 8) {
-                float e[8], b[8];
-#pragma unroll
-                for (uint32_t t = 0; t < 8; t++) {
-                    uint32_t cj = lane_value(cf, j + t);
-                    b[t] = lane_value(beta, j + t);
-                    e[t] = live ? w.cfg_emb[(size_t)cj * pool + k] : 0.0f;
-                }
-#pragma unroll
-                for (uint32_t t = 0; t < 8; t++) acc += b[t] * e[t];
+            const uint32_t left = n - c0, cn = index(c0 + 64);
+            const float bn = belief(c0 + 64);
+            if (left > 16) fetch(e1, cf, 16);
+            add(e0, beta, 0, left);
+            if (left > 16) {
+                if (left > 32) fetch(e0, cf, 32);
+                add(e1, beta, 16, left - 16);
             }
-            for (; j < m; j++) {
-                uint32_t cj = lane_value(cf, j);
-                float e = live ? w.cfg_emb[(size_t)cj * pool + k] : 0.0f;
-                acc += lane_value(beta, j) * e;
+            if (left > 32) {
+                if (left > 48) fetch(e1, cf, 48);
+                add(e0, beta, 32, left - 32);
             }
+            if (left > 48) {
+                if (left > 64) fetch(e0, cn, 0);
+                add(e1, beta, 48, left - 48);
+            }
+            cf = cn;
+            beta = bn;
         }
         if (live) {
             own[(size_t)row * in + k] = acc;
@@ -516,38 +550,123 @@ __global__ __launch_bounds__(BLOCK) void k_pool_exact(WaveDev w, int player, flo
     }
 }
 
-// 16-bit nets: one wavefront per pool group (up to POOL_GROUP rows of one
-// player whose configs are the same list), on the f32 MFMA. With A the
-// group's reach rows (row 15: ones) and B the configs' embeddings, four
-// 16x16x4 products per 4 configs accumulate U[r][k] = sum_c reach_r(c) e_c(k)
-// and, in row 15, S[k] = sum_c e_c(k); each row's mass is summed on the VALU
-// from the same reach values. Then pooled = U / mass, or S / n where
-// the mass is below the smoothing floor (the uniform weights of
-// normalize_weights). Each config's embedding is read once for the group.
-// Products are exact f32; only the summation order differs from the CPU's,
-// far below the 16-bit rounding of the stored query input.
+// 16-bit nets: pool groups (up to POOL_GROUP rows of one player whose configs
+// are the same list) on the f32 MFMA. With A the group's reach rows (row 15:
+// ones) and B the configs' embeddings, a 16x16x4 product per 16 dimensions and
+// 4 configs accumulates U[r][k] = sum_c reach_r(c) e_c(k) and, in row 15, S[k]
+// = sum_c e_c(k); each row's mass is summed on the VALU from the same reach
+// values. Then pooled = U / mass, or S / n where the mass is below the
+// smoothing floor (the uniform weights of normalize_weights). Each config's
+// embedding is read once for the group. Products are exact f32; only the
+// summation order differs from the CPU's, far below the 16-bit rounding of the
+// stored query input.
+//
+// A list of up to POOL_LONG configs takes one wavefront, all its loads of a
+// 64-config chunk in flight together. A longer one is a chain of chunks, each
+// with dependent loads (config indices, then embeddings), so it takes a whole
+// workgroup: the wavefronts split the dimensions (16 each, so that every sum
+// keeps its one order), share the reach and the indices through LDS, and the
+// next chunk's are on their way while the current one multiplies. Bound: the
+// latency of those loads with four wavefronts per SIMD (five spill). Leaf-input
+// time per wave, all lists on single wavefronts against long ones on
+// workgroups: 32 heavy-tailed subgames 12.0 -> 8.4 ms, 64 depth-1 subgames in
+// compensated f16 2.43 -> 1.35 ms, 256 depth-2 subgames 3.81 -> 3.61 ms.
+
+// Configs past which a list takes a workgroup (256 depth-2 subgames: 3.74 ms
+// per wave from 128 on, 3.61 from 192, 3.75 from 256; below the line four
+// wavefronts wait for the loads of one or two chunks), and configs per LDS
+// chunk.
+constexpr uint32_t POOL_LONG = 192, POOL_CH = 64;
+// A chunk's reach rows in LDS: config c of a row at POOL_Q (c % 4) + c / 4, so
+// that a lane's configs of four consecutive MFMA steps are one 16-byte read;
+// the pitches spread a wavefront's reads and writes over the banks.
+constexpr uint32_t POOL_Q = 48, POOL_ROW = 4 * POOL_Q + 4;
+// A finished group in LDS as 16-bit operands: rows of 64 dimensions.
+constexpr uint32_t POOL_OUT = 72;
+
+struct PoolLds {
+    union {
+        struct {
+            float a[2][POOL_GROUP][POOL_ROW];
+            uint32_t idx[2][4][POOL_CH / 4];  // config c at [c % 4][c / 4]
+        } chunk;
+        uint16_t out[BLOCK / 64][2][POOL_GROUP + 1][POOL_OUT];  // per wavefront (short lists) and plane
+    };
+    uint32_t rbase[POOL_GROUP];
+};
+
+// Writes a group's pooled rows (the 64 dimensions from k0 on, row rr at
+// src[rr], the compensated lo plane at src[16 + rr]) into both query inputs,
+// eight dimensions per store: n threads, this one the t-th.
 template <int PREC>
-__global__ __launch_bounds__(BLOCK) void k_pool_mfma(WaveDev w, int player, uint16_t* x0, uint16_t* x1, int acc,
-                                                   float ds, uint32_t pool_blocks) {
-    uint32_t pbk;
-    if (accumulate_blocks(w, acc, ds, pool_blocks, &pbk)) return;
-    uint32_t g = __builtin_amdgcn_readfirstlane((pbk * blockDim.x + threadIdx.x) >> 6);
-    const uint32_t lane = threadIdx.x & 63;
-    uint32_t p = player < 0 ? 0u : (uint32_t)player;
-    if (player < 0 && g >= w.npool[0]) {
-        g -= w.npool[0];
-        p = 1;
+__device__ __forceinline__ void pool_store(const WaveDev& w, const PoolGroup* grp, uint32_t p, uint16_t* x0,
+                                           uint16_t* x1, const uint16_t (*src)[POOL_OUT], uint32_t k0, uint32_t t,
+                                           uint32_t n) {
+    uint16_t* own = p ? x1 : x0;    // pooled_p is the first block of traverser p's query
+    uint16_t* other = p ? x0 : x1;  // and the second block of the other traverser's
+    const uint32_t G = grp->nrows, pool = w.pool;
+    if (pool % 8 == 0) {
+        for (uint32_t e = t; e < G * 8; e += n) {
+            const uint32_t rr = e >> 3, k = k0 + 8 * (e & 7);
+            if (k >= pool) continue;
+            const uint32_t row = grp->row[rr];
+            const size_t o = frag_off(row, k, w.in), x = frag_off(row, pool + k, w.in);
+            const uint4 hi = *(const uint4*)&src[rr][k - k0];
+            *(uint4*)(own + o) = hi;
+            *(uint4*)(other + x) = hi;
+            if (PREC == WC_F16X) {
+                const uint4 lo = *(const uint4*)&src[POOL_GROUP + 1 + rr][k - k0];
+                *(uint4*)(own + o + w.xplane) = lo;
+                *(uint4*)(other + x + w.xplane) = lo;
+            }
+        }
+        return;
     }
-    if (g >= w.npool[p]) return;  // wave-uniform
-    const PoolGroup* grp = w.pool_grp[p] + g;
+    for (uint32_t e = t; e < G * 64; e += n) {
+        const uint32_t rr = e >> 6, k = k0 + (e & 63);
+        if (k >= pool) continue;
+        const uint32_t row = grp->row[rr];
+        const size_t o = frag_off(row, k, w.in), x = frag_off(row, pool + k, w.in);
+        own[o] = other[x] = src[rr][k - k0];
+        if (PREC == WC_F16X) own[o + w.xplane] = other[x + w.xplane] = src[POOL_GROUP + 1 + rr][k - k0];
+    }
+}
+
+// One 16-dimension tile's sums (this lane: rows 4q .. 4q + 3, dimension d of
+// the 64) over their rows' masses, into the group's LDS rows.
+template <int PREC>
+__device__ __forceinline__ void pool_tile(const float4v& acc, const float (&tot)[4], float inv_n, uint32_t q,
+                                          uint32_t i, uint32_t d, uint16_t (*dst)[POOL_OUT]) {
+    const float S = __shfl(acc[3], (int)(48 + i), 64);  // row 15 of this column
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+        const float y = tot[v] > SMOOTHF ? acc[v] * (1.0f / tot[v]) : S * inv_n;
+        const uint32_t rr = 4 * q + v;  // (row 15's slot is never stored)
+        store_operand<PREC>(dst, rr * POOL_OUT + d, y, (POOL_GROUP + 1) * POOL_OUT);
+    }
+}
+
+// Row i's mass from the lanes' partial sums (lanes i, i + 16, i + 32, i + 48),
+// to the masses of rows 4q .. 4q + 3; returns row i's.
+__device__ __forceinline__ float pool_mass(float tpart, uint32_t q, float (&tot)[4]) {
+    float ti = tpart + __shfl_xor(tpart, 16, 64);
+    ti += __shfl_xor(ti, 32, 64);
+#pragma unroll
+    for (int v = 0; v < 4; v++) tot[v] = __shfl(ti, (int)(4 * q + v), 64);
+    return ti;
+}
+
+// A short list: one wavefront.
+template <int PREC>
+__device__ __forceinline__ void pool_short(const WaveDev& w, const PoolGroup* grp, uint32_t p, uint16_t* x0,
+                                           uint16_t* x1, uint16_t (*dst)[POOL_OUT]) {
+    const uint32_t lane = threadIdx.x & 63;
     const uint32_t n = grp->n, G = grp->nrows;
     const uint32_t i = lane & 15, q = lane >> 4;  // A row / B column, and config within a 4-step
     const float* ra = w.reach + grp->rbase[i < POOL_GROUP ? i : 0];  // lane row 15 reads no reach
     const float aconst = i == 15 ? 1.0f : 0.0f;  // rows G..14 are zero, row 15 sums the embeddings
     const uint32_t* cfgs = w.row_cfg + grp->cfg;
-    const uint32_t pool = w.pool, in = w.in;
-    uint16_t* own = p ? x1 : x0;
-    uint16_t* other = p ? x0 : x1;
+    const uint32_t pool = w.pool;
     float tot[4] = {0.0f, 0.0f, 0.0f, 0.0f};  // mass of rows 4q .. 4q + 3
     for (uint32_t k0 = 0; k0 < pool; k0 += 64) {
         float4v acc[4];
@@ -595,30 +714,130 @@ __global__ __launch_bounds__(BLOCK) void k_pool_mfma(WaveDev w, int player, uint
             }
         }
         if (k0 == 0) {
-            // Row i's mass: lanes i, i + 16, i + 32, i + 48 hold its partial sums.
-            float ti = tpart + __shfl_xor(tpart, 16, 64);
-            ti += __shfl_xor(ti, 32, 64);
-#pragma unroll
-            for (int v = 0; v < 4; v++) tot[v] = __shfl(ti, (int)(4 * q + v), 64);
+            const float ti = pool_mass(tpart, q, tot);
             if (q == 0 && i < G) w.mass[2 * grp->row[i] + p] = ti;
         }
         const float inv_n = 1.0f / (float)(n > 0 ? n : 1);
 #pragma unroll
-        for (int t = 0; t < 4; t++) {
-            const float S = __shfl(acc[t][3], (int)(48 + i), 64);  // row 15 of this column
-            const uint32_t k = k0 + 16 * t + i;
-            if (!kl[t]) continue;
-#pragma unroll
-            for (int v = 0; v < 4; v++) {
-                const uint32_t rr = 4 * q + v;
-                if (rr >= G) continue;
-                const float y = tot[v] > SMOOTHF ? acc[t][v] * (1.0f / tot[v]) : S * inv_n;
-                const uint32_t row = grp->row[rr];
-                store_operand<PREC>(own, frag_off(row, k, in), y, w.xplane);
-                store_operand<PREC>(other, frag_off(row, pool + k, in), y, w.xplane);
-            }
-        }
+        for (int t = 0; t < 4; t++) pool_tile<PREC>(acc[t], tot, inv_n, q, i, 16 * t + i, dst);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // the wavefront's own LDS rows
+        pool_store<PREC>(w, grp, p, x0, x1, dst, k0, lane, 64);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     }
+}
+
+// A long list: the workgroup, one 16-dimension tile per wavefront.
+template <int PREC>
+__device__ __forceinline__ void pool_long(const WaveDev& w, const PoolGroup* grp, uint32_t p, uint16_t* x0,
+                                          uint16_t* x1, PoolLds& sh) {
+    const uint32_t t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const uint32_t n = grp->n, G = min(grp->nrows, POOL_GROUP);
+    const uint32_t i = lane & 15, q = lane >> 4;
+    const uint32_t* cfgs = w.row_cfg + grp->cfg;
+    const uint32_t pool = w.pool;
+    if (t < POOL_GROUP) sh.rbase[t] = grp->rbase[t];
+    __syncthreads();
+    // One chunk: POOL_CH indices, and G x POOL_CH reach values, 8 per thread.
+    constexpr int PER = (POOL_GROUP * POOL_CH + BLOCK - 1) / BLOCK;
+    float rv[PER];
+    uint32_t iv = 0xffffffffu;
+    const uint32_t cc = t % POOL_CH, r0 = t / POOL_CH;  // this thread's column, and its rows r0, r0 + 2, ...
+    auto fetch = [&](uint32_t c0) {
+        const uint32_t c = c0 + cc;
+        if (t < POOL_CH) iv = c < n ? cfgs[c] : 0xffffffffu;
+#pragma unroll
+        for (int j = 0; j < PER; j++) {
+            const uint32_t r = r0 + j * (BLOCK / POOL_CH);
+            rv[j] = r < G && c < n ? w.reach[sh.rbase[r] + c] : 0.0f;
+        }
+    };
+    auto stage = [&](int buf) {
+        if (t < POOL_CH) sh.chunk.idx[buf][cc & 3][cc >> 2] = iv;
+#pragma unroll
+        for (int j = 0; j < PER; j++) {
+            const uint32_t r = r0 + j * (BLOCK / POOL_CH);
+            if (r < G) sh.chunk.a[buf][r][POOL_Q * (cc & 3) + (cc >> 2)] = rv[j];
+        }
+    };
+    float tot[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (uint32_t k0 = 0; k0 < pool; k0 += 64) {
+        const uint32_t k = k0 + 16 * wave + i;
+        const bool kl = k < pool;
+        const float* emb = w.cfg_emb + (kl ? k : 0u);
+        float4v acc = float4v{0.0f, 0.0f, 0.0f, 0.0f};
+        float tpart = 0.0f;
+        fetch(0);
+        stage(0);
+        __syncthreads();
+        int buf = 0;
+        for (uint32_t c0 = 0; c0 < n; c0 += POOL_CH, buf ^= 1) {
+            const bool more = c0 + POOL_CH < n;
+            float b[POOL_CH / 4];
+#pragma unroll
+            for (int s4 = 0; s4 < (int)POOL_CH / 16; s4++) {
+                const uint4 cf = *(const uint4*)&sh.chunk.idx[buf][q][4 * s4];
+                const uint32_t f[4] = {cf.x, cf.y, cf.z, cf.w};
+#pragma unroll
+                for (int s = 0; s < 4; s++) {
+                    const bool live = f[s] != 0xffffffffu && kl;
+                    const float e = emb[(size_t)(live ? f[s] : 0u) * pool];
+                    b[4 * s4 + s] = live ? e : 0.0f;
+                }
+            }
+            if (more) fetch(c0 + POOL_CH);
+#pragma unroll
+            for (int s4 = 0; s4 < (int)POOL_CH / 16; s4++) {
+                if (c0 + 16 * s4 >= n) break;  // block-uniform
+                float4v a4 = *(const float4v*)&sh.chunk.a[buf][i < POOL_GROUP ? i : 0][POOL_Q * q + 4 * s4];
+#pragma unroll
+                for (int s = 0; s < 4; s++) {
+                    const uint32_t c = c0 + 4 * (4 * s4 + s) + q;
+                    const float a = i < G ? a4[s] : i == 15 && c < n ? 1.0f : 0.0f;
+                    tpart += a;
+                    if (c0 + 4 * (4 * s4 + s) < n) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a, b[4 * s4 + s], acc, 0, 0, 0);
+                }
+            }
+            if (more) stage(buf ^ 1);
+            __syncthreads();
+        }
+        if (k0 == 0) {
+            const float ti = pool_mass(tpart, q, tot);
+            if (wave == 0 && q == 0 && i < G) w.mass[2 * grp->row[i] + p] = ti;
+        }
+        pool_tile<PREC>(acc, tot, 1.0f / (float)n, q, i, 16 * wave + i, sh.out[0][0]);  // (the chunks are done)
+        __syncthreads();
+        pool_store<PREC>(w, grp, p, x0, x1, sh.out[0][0], k0, t, BLOCK);
+        __syncthreads();
+    }
+}
+
+template <int PREC>
+__global__ __launch_bounds__(BLOCK, 4) void k_pool_mfma(WaveDev w, int player, uint16_t* x0, uint16_t* x1, int acc,
+                                                   float ds, uint32_t pool_blocks) {
+    __shared__ __attribute__((aligned(16))) PoolLds sh;
+    uint32_t pbk;
+    if (accumulate_blocks(w, acc, ds, pool_blocks, &pbk)) return;
+    // One workgroup per long list (each player's lists come longest first),
+    // then a wavefront per short one.
+    const uint32_t l0 = player != 1 ? w.nlong[0] : 0, l1 = player != 0 ? w.nlong[1] : 0;
+    if (pbk < l0 + l1) {
+        const uint32_t p = pbk < l0 ? 0 : 1;
+        pool_long<PREC>(w, w.pool_grp[p] + (p ? pbk - l0 : pbk), p, x0, x1, sh);
+        return;
+    }
+    const uint32_t wave = threadIdx.x >> 6;
+    uint32_t g = __builtin_amdgcn_readfirstlane((pbk - l0 - l1) * (BLOCK / 64) + wave);
+    const uint32_t s0 = player != 1 ? w.npool[0] - w.nlong[0] : 0;
+    const uint32_t p = g < s0 ? 0 : 1;
+    g = p ? g - s0 + w.nlong[1] : g + w.nlong[0];
+    if (player == 0 ? p == 1 : g >= w.npool[1] && p == 1) return;  // wave-uniform: past the last group
+    pool_short<PREC>(w, w.pool_grp[p] + g, p, x0, x1, sh.out[wave][0]);
+}
+
+uint32_t pool_long_groups(const PoolGroup* grp, uint32_t n) {
+    uint32_t k = 0;
+    while (k < n && grp[k].n > POOL_LONG) k++;
+    return k;
 }
 
 void launch_pool(const WaveDev& w, int player, int precision, void* x0, void* x1, hipStream_t s, int acc,
@@ -627,13 +846,22 @@ void launch_pool(const WaveDev& w, int player, int precision, void* x0, void* x1
     if (precision == WC_PRECISE) {
         size_t waves = (size_t)w.rows * (player < 0 ? 2 : 1);
         const uint32_t pb = grid_for(waves * 64);
-        if (pb + accb)
-            hipLaunchKernelGGL(k_pool_exact, dim3(pb + accb), dim3(BLOCK), 0, s, w, player, (float*)x0, (float*)x1,
-                               acc, ds, pb);
+        if (!(pb + accb)) return;
+        if (w.emb_wide)
+            hipLaunchKernelGGL(k_pool_exact<true>, dim3(pb + accb), dim3(BLOCK), 0, s, w, player, (float*)x0,
+                               (float*)x1, acc, ds, pb);
+        else
+            hipLaunchKernelGGL(k_pool_exact<false>, dim3(pb + accb), dim3(BLOCK), 0, s, w, player, (float*)x0,
+                               (float*)x1, acc, ds, pb);
         return;
     }
-    size_t waves = player < 0 ? (size_t)w.npool[0] + w.npool[1] : w.npool[player];
-    const uint32_t pb = grid_for(waves * 64);
+    size_t waves = 0, wide = 0;
+    for (int p = 0; p < 2; p++)
+        if (player < 0 || p == player) {
+            wide += w.nlong[p];
+            waves += w.npool[p] - w.nlong[p];
+        }
+    const uint32_t pb = (uint32_t)wide + grid_for(waves * 64);
     if (!(pb + accb)) return;
     dim3 g(pb + accb);
     if (precision == WC_F16)
