@@ -90,63 +90,98 @@ void launch_seed_reach(const WaveDev& w, float* reach, size_t reach_len, int roo
     hipLaunchKernelGGL(k_seed_reach, dim3(w.ntrees), dim3(BLOCK), 0, s, w, reach, root_index);
 }
 
-// Row elements are handled ROW_BATCH at a time: a batch's loads are issued
-// together (indices, then the values they name) and its part of the reduction
-// is taken after, in element order, so every sum keeps the CPU's order.
-constexpr uint32_t ROW_BATCH = 12;   // value rows: decision rows up to 12 actions in one pass
-constexpr uint32_t REACH_BATCH = 8;  // reach gathers and average accumulation
+// A row's elements are contiguous and few (2 to 6 on average, rarely over 8),
+// so they are taken four at a time with no branch per element: one 16-byte
+// load per array and four elements (element arrays are readable 12 bytes past
+// their end: another section of the same allocation follows), elements past
+// the row's end redirected to an index that is valid, their terms dropped by a
+// select. Every sum keeps the CPU's order. A branch per element costs ten
+// instructions on top of what it guards, and these kernels were bound by them
+// (3,400 instructions in the sweep, 400 of them exec-mask saves): per launch,
+// branches per element against quads, the sweep 66 -> 55 us and the reach 57 ->
+// 45 us on 256 depth-2 subgames, 53 -> 41 and 53 -> 41 us on 32 heavy-tailed
+// ones, 21.7 -> 14.5 and 14.5 -> 12 us on a single depth-1 subgame; top regions
+// 69 -> 67 us per iteration (their launches set the time).
+__device__ __forceinline__ void quad(const uint32_t* p, uint32_t (&v)[4]) { __builtin_memcpy(v, p, 16); }
+__device__ __forceinline__ void quad(const float* p, float (&v)[4]) { __builtin_memcpy(v, p, 16); }
+// A wave-uniform pointer, held in scalar registers: a lane's choice between two
+// kernel arguments would otherwise become a choice of where to load the
+// pointer from, one dependent load more.
+template <class T>
+__device__ __forceinline__ T* scalar(T* p) {
+    asm("" : "+s"(p));
+    return p;
+}
+// The first n (at least 1) of four elements.
+__device__ __forceinline__ void store_quad(float* p, const float (&v)[4], uint32_t n) {
+    if (n >= 4) {
+        __builtin_memcpy(p, v, 16);
+        return;
+    }
+    p[0] = v[0];
+    if (n > 1) p[1] = v[1];
+    if (n > 2) p[2] = v[2];
+}
+
+constexpr uint32_t ROW_QUADS = 3;   // decision rows up to 12 actions stay in registers
+constexpr uint32_t ROW_BATCH = 12;  // longer ones go 12 actions at a time
 // Network-leaf slots in flight per thread in the sweep's leaf phase.
 constexpr uint32_t LEAF_BATCH = 4;
 
 // One child config's reach: the reverse gather in stored order (the CPU's
 // scatter order, engine/src/serialize.rs:714-723). With LDSR the unit's reach
 // window [rw, rw + rn) is also kept in LDS at lr: parent reach inside it is
-// read from there, and the row's result goes to both.
+// read from there (a parent's slots are all inside or all outside), and the
+// row's result goes to both.
+template <bool REV, bool INSIDE>
+__device__ __forceinline__ float reach_sum(const WaveDev& w, const float* reach, const float* strat, uint32_t lo,
+                                           uint32_t n, uint32_t base) {
+    const uint32_t* esrc = (REV ? w.rev_src : w.rvd_src) + lo;
+    const uint32_t* ecell = w.rev_cell + (REV ? lo : 0);
+    const float* ep = w.rvd_p + (REV ? 0 : lo);
+    float v = 0.0f;
+    for (uint32_t c0 = 0; c0 < n; c0 += 8) {
+        const bool two = n - c0 > 4;
+        uint32_t src[2][4], cell[2][4];
+        float a[2][4], b[2][4];
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+            if (h == 0 || two) {
+                quad(esrc + c0 + 4 * h, src[h]);
+                if (REV)
+                    quad(ecell + c0 + 4 * h, cell[h]);
+                else
+                    quad(ep + c0 + 4 * h, b[h]);
+            }
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+            if (h == 0 || two)
+#pragma unroll
+                for (uint32_t k = 0; k < 4; k++) {
+                    const bool in = c0 + 4 * h + k < n;
+                    a[h][k] = reach[in ? base + src[h][k] : base];
+                    if (REV) b[h][k] = strat[in ? cell[h][k] : 0u];
+                }
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+            if (h == 0 || two)
+#pragma unroll
+                for (uint32_t k = 0; k < 4; k++) v = c0 + 4 * h + k < n ? v + a[h][k] * b[h][k] : v;
+    }
+    return v;
+}
 template <bool LDSR = false>
 __device__ __forceinline__ void reach_row(const WaveDev& w, float* reach, const float* strat, ReachRec q,
                                           float* lr = nullptr, uint32_t rw = 0, uint32_t rn = 0) {
-    const uint32_t lo = q.start, n = q.kn & REC_N, base = q.pbase;
-    auto parent = [&](uint32_t i) { return LDSR && i - rw < rn ? lr[i - rw] : reach[i]; };
-    float v = 0.0f;
-    if ((q.kn >> 31) == REACH_REV) {
-        for (uint32_t c0 = 0; c0 < n; c0 += REACH_BATCH) {
-            const uint32_t m = n - c0 < REACH_BATCH ? n - c0 : REACH_BATCH;
-            uint32_t src[REACH_BATCH], cell[REACH_BATCH];
-            float a[REACH_BATCH], b[REACH_BATCH];
-#pragma unroll
-            for (uint32_t k = 0; k < REACH_BATCH; k++)
-                if (k < m) {
-                    src[k] = w.rev_src[lo + c0 + k];
-                    cell[k] = w.rev_cell[lo + c0 + k];
-                }
-#pragma unroll
-            for (uint32_t k = 0; k < REACH_BATCH; k++)
-                if (k < m) {
-                    a[k] = parent(base + src[k]);
-                    b[k] = strat[cell[k]];
-                }
-#pragma unroll
-            for (uint32_t k = 0; k < REACH_BATCH; k++)
-                if (k < m) v += a[k] * b[k];
-        }
+    const uint32_t lo = q.start, n = q.kn & REC_N;
+    const bool rev = (q.kn >> 31) == REACH_REV;
+    float v;
+    if (LDSR && q.pbase - rw < rn) {
+        const uint32_t base = q.pbase - rw;
+        v = rev ? reach_sum<true, true>(w, lr, strat, lo, n, base) : reach_sum<false, true>(w, lr, strat, lo, n, base);
     } else {
-        for (uint32_t c0 = 0; c0 < n; c0 += REACH_BATCH) {
-            const uint32_t m = n - c0 < REACH_BATCH ? n - c0 : REACH_BATCH;
-            uint32_t src[REACH_BATCH];
-            float a[REACH_BATCH], pr[REACH_BATCH];
-#pragma unroll
-            for (uint32_t k = 0; k < REACH_BATCH; k++)
-                if (k < m) {
-                    src[k] = w.rvd_src[lo + c0 + k];
-                    pr[k] = w.rvd_p[lo + c0 + k];
-                }
-#pragma unroll
-            for (uint32_t k = 0; k < REACH_BATCH; k++)
-                if (k < m) a[k] = parent(base + src[k]);
-#pragma unroll
-            for (uint32_t k = 0; k < REACH_BATCH; k++)
-                if (k < m) v += a[k] * pr[k];
-        }
+        v = rev ? reach_sum<true, false>(w, reach, strat, lo, n, q.pbase)
+                : reach_sum<false, false>(w, reach, strat, lo, n, q.pbase);
     }
     reach[q.out] = v;
     if (LDSR) lr[q.out - rw] = v;
@@ -158,19 +193,25 @@ __device__ __forceinline__ void reach_row(const WaveDev& w, float* reach, const 
 // the same two rounded steps in the same order, taken in one pass.
 __device__ __forceinline__ void accumulate_row(const WaveDev& w, AccRec q, float ds) {
     const float r = w.reach[q.ridx];
-    const uint32_t lo = q.lo, n = q.n;
-    for (uint32_t c0 = 0; c0 < n; c0 += REACH_BATCH) {
-        const uint32_t m = n - c0 < REACH_BATCH ? n - c0 : REACH_BATCH;
-        float cu[REACH_BATCH], sm[REACH_BATCH];
+    const uint32_t n = q.n;
+    const float* cur = w.cur + q.lo;
+    float* sum = w.sum + q.lo;
+    for (uint32_t c0 = 0; c0 < n; c0 += 8) {
+        const bool two = n - c0 > 4;
+        float cu[2][4], sm[2][4];
 #pragma unroll
-        for (uint32_t j = 0; j < REACH_BATCH; j++)
-            if (j < m) {
-                cu[j] = w.cur[lo + c0 + j];
-                sm[j] = w.sum[lo + c0 + j];
+        for (int h = 0; h < 2; h++)
+            if (h == 0 || two) {
+                quad(cur + c0 + 4 * h, cu[h]);
+                quad(sum + c0 + 4 * h, sm[h]);
             }
 #pragma unroll
-        for (uint32_t j = 0; j < REACH_BATCH; j++)
-            if (j < m) w.sum[lo + c0 + j] = sm[j] * ds + r * cu[j];
+        for (int h = 0; h < 2; h++)
+            if (h == 0 || two) {
+#pragma unroll
+                for (int k = 0; k < 4; k++) sm[h][k] = sm[h][k] * ds + r * cu[h][k];
+                store_quad(sum + c0 + 4 * h, sm[h], n - c0 - 4 * h);
+            }
     }
 }
 
@@ -926,46 +967,34 @@ __device__ __forceinline__ void backprop_row(const WaveDev& w, int p, BackRec q,
         if (LDSV) lv[i - vw] = v;
     };
     const uint32_t kind = q.kn >> 30, n = q.kn & REC_N, lo = q.start;
-    if (kind == BACK_DRAW) {  // the traverser draws: push values through the outcome row
-        const uint32_t cb = q.arg;
+    if (kind != BACK_OWN) {
+        // The traverser draws: push values through the outcome row. The
+        // opponent decides: sum the children in child order.
+        const bool draw = kind == BACK_DRAW;
+        const uint32_t* eto = (draw ? scalar(w.draw_to) : scalar(p ? w.child_vb[1] : w.child_vb[0])) + lo;
+        const float* ep = w.draw_p + (draw ? lo : 0);
         float v = 0.0f;
-        for (uint32_t c0 = 0; c0 < n; c0 += ROW_BATCH) {
-            const uint32_t m = n - c0 < ROW_BATCH ? n - c0 : ROW_BATCH;
-            uint32_t to[ROW_BATCH];
-            float pr[ROW_BATCH], cv[ROW_BATCH];
+        for (uint32_t c0 = 0; c0 < n; c0 += 8) {
+            const bool two = n - c0 > 4;
+            uint32_t to[2][4];
+            float pr[2][4], cv[2][4];
 #pragma unroll
-            for (uint32_t k = 0; k < ROW_BATCH; k++)
-                if (k < m) {
-                    to[k] = w.draw_to[lo + c0 + k];
-                    pr[k] = w.draw_p[lo + c0 + k];
+            for (int h = 0; h < 2; h++)
+                if (h == 0 || two) {
+                    quad(eto + c0 + 4 * h, to[h]);
+                    if (draw) quad(ep + c0 + 4 * h, pr[h]);
                 }
 #pragma unroll
-            for (uint32_t k = 0; k < ROW_BATCH; k++)
-                if (k < m) cv[k] = get(cb + to[k]);
+            for (int h = 0; h < 2; h++)
+                if (h == 0 || two)
 #pragma unroll
-            for (uint32_t k = 0; k < ROW_BATCH; k++)
-                if (k < m) v += pr[k] * cv[k];
-        }
-        put(q.out, v);
-        return;
-    }
-    if (kind == BACK_OPP) {  // opponent decision: sum the children in child order
-        const uint32_t c = q.arg;
-        const uint32_t* cvb = w.child_vb[p] + lo;
-        float v = 0.0f;
-        for (uint32_t c0 = 0; c0 < n; c0 += ROW_BATCH) {
-            const uint32_t m = n - c0 < ROW_BATCH ? n - c0 : ROW_BATCH;
-            uint32_t cb[ROW_BATCH];
-            float cv[ROW_BATCH];
+                    for (uint32_t k = 0; k < 4; k++) cv[h][k] = get(c0 + 4 * h + k < n ? q.arg + to[h][k] : q.out);
 #pragma unroll
-            for (uint32_t k = 0; k < ROW_BATCH; k++)
-                if (k < m) cb[k] = cvb[c0 + k];
+            for (int h = 0; h < 2; h++)
+                if (h == 0 || two)
 #pragma unroll
-            for (uint32_t k = 0; k < ROW_BATCH; k++)
-                if (k < m) cv[k] = get(cb[k] + c);
-#pragma unroll
-            for (uint32_t k = 0; k < ROW_BATCH; k++)
-                if (k < m) v += cv[k];
+                    for (uint32_t k = 0; k < 4; k++)
+                        v = c0 + 4 * h + k < n ? v + (draw ? pr[h][k] * cv[h][k] : cv[h][k]) : v;
         }
         put(q.out, v);
         return;
@@ -976,41 +1005,62 @@ __device__ __forceinline__ void backprop_row(const WaveDev& w, int p, BackRec q,
     // predict delta, EPS), normalised by a reciprocal multiply. The sum's
     // discount (sum *= ds) is taken with the accumulation in the reach sweep.
     const float* st = MODE == MODE_VALUE ? strat : w.cur;
-    if (n <= ROW_BATCH) {  // one batch: everything stays in registers
-        uint32_t lvi[ROW_BATCH];
-        float sv[ROW_BATCH], qv[ROW_BATCH], old[ROW_BATCH];
+    if (n <= ROW_BATCH) {  // everything stays in registers
+        uint32_t lvi[ROW_QUADS][4];
+        float sv[ROW_QUADS][4], qv[ROW_QUADS][4], old[ROW_QUADS][4];
+        const bool more[ROW_QUADS] = {true, n > 4, n > 8};
 #pragma unroll
-        for (uint32_t k = 0; k < ROW_BATCH; k++)
-            if (k < n) {
-                lvi[k] = w.legal_value[lo + k];
-                sv[k] = st[lo + k];
-                if (MODE == MODE_REGRET) old[k] = w.regret[lo + k];
+        for (uint32_t h = 0; h < ROW_QUADS; h++)
+            if (more[h]) {
+                quad(w.legal_value + lo + 4 * h, lvi[h]);
+                quad(st + lo + 4 * h, sv[h]);
+                if (MODE == MODE_REGRET) quad(w.regret + lo + 4 * h, old[h]);
             }
+        // A cell past the row's end is like one without a successor, then not stored.
 #pragma unroll
-        for (uint32_t k = 0; k < ROW_BATCH; k++)
-            if (k < n) qv[k] = lvi[k] != 0xffffffffu ? get(lvi[k]) : 0.0f;
+        for (uint32_t h = 0; h < ROW_QUADS; h++)
+            if (more[h])
+#pragma unroll
+                for (uint32_t k = 0; k < 4; k++) {
+                    if (4 * h + k >= n) lvi[h][k] = 0xffffffffu;
+                    const bool live = lvi[h][k] != 0xffffffffu;
+                    const float x = get(live ? lvi[h][k] : q.out);
+                    qv[h][k] = live ? x : 0.0f;
+                }
         float base = 0.0f;
 #pragma unroll
-        for (uint32_t k = 0; k < ROW_BATCH; k++)
-            if (k < n && lvi[k] != 0xffffffffu) base += qv[k] * sv[k];
+        for (uint32_t h = 0; h < ROW_QUADS; h++)
+            if (more[h])
+#pragma unroll
+                for (uint32_t k = 0; k < 4; k++)
+                    base = lvi[h][k] != 0xffffffffu ? base + qv[h][k] * sv[h][k] : base;
         put(q.out, base);
         if (MODE == MODE_VALUE) return;
-        float total = 0.0f, v[ROW_BATCH];
+        float total = 0.0f;
 #pragma unroll
-        for (uint32_t k = 0; k < ROW_BATCH; k++)
-            if (k < n) {
-                float delta = 0.0f;
-                if (lvi[k] != 0xffffffffu) delta += qv[k];
-                delta -= base;
-                float r = old[k] * (old[k] > 0.0f ? da : db) + delta;
-                w.regret[lo + k] = r;
-                v[k] = fmaxf(r + predict * delta, EPSF);
-                total += v[k];
+        for (uint32_t h = 0; h < ROW_QUADS; h++)
+            if (more[h]) {
+#pragma unroll
+                for (uint32_t k = 0; k < 4; k++) {
+                    float delta = 0.0f;
+                    delta += qv[h][k];  // (zero without a successor)
+                    delta -= base;
+                    const float r = old[h][k] * (old[h][k] > 0.0f ? da : db) + delta;
+                    old[h][k] = r;
+                    sv[h][k] = fmaxf(r + predict * delta, EPSF);
+                    total = 4 * h + k < n ? total + sv[h][k] : total;
+                }
+                store_quad(w.regret + lo + 4 * h, old[h], n - 4 * h);
             }
-        float inv = total > 0.0f ? 1.0f / total : 1.0f;
+        const bool pos = total > 0.0f;
+        const float inv = pos ? 1.0f / total : 1.0f;
 #pragma unroll
-        for (uint32_t k = 0; k < ROW_BATCH; k++)
-            if (k < n) w.cur[lo + k] = total > 0.0f ? v[k] * inv : v[k];
+        for (uint32_t h = 0; h < ROW_QUADS; h++)
+            if (more[h]) {
+#pragma unroll
+                for (uint32_t k = 0; k < 4; k++) sv[h][k] = pos ? sv[h][k] * inv : sv[h][k];
+                store_quad(w.cur + lo + 4 * h, sv[h], n - 4 * h);
+            }
         return;
     }
     // Longer rows: the same arithmetic in three batched passes (base; update,
@@ -1101,21 +1151,19 @@ __global__ __launch_bounds__(BLOCK) void k_sweep(WaveDev w, uint32_t unit0, cons
     BackRec q{};
     if (l && b + t < e) q = back[b + t];
     // Network leaves: one value slot per thread, LEAF_BATCH slots per thread
-    // in flight (their records, then the values they name).
+    // in flight (their records, then the values they name; slots past the end
+    // repeat the last and are not stored).
+    const LeafRec* leaves = w.leaf_rec[p];
     for (uint32_t k0 = leaf0; k0 < leaf1; k0 += LEAF_BATCH * BLOCK) {
         LeafRec lr[LEAF_BATCH];
         float h[LEAF_BATCH], m[LEAF_BATCH];
 #pragma unroll
-        for (uint32_t j = 0; j < LEAF_BATCH; j++) {
-            const uint32_t k = k0 + j * BLOCK + threadIdx.x;
-            if (k < leaf1) lr[j] = w.leaf_rec[p][k];
-        }
+        for (uint32_t j = 0; j < LEAF_BATCH; j++) lr[j] = leaves[min(k0 + j * BLOCK + threadIdx.x, leaf1 - 1)];
 #pragma unroll
-        for (uint32_t j = 0; j < LEAF_BATCH; j++)
-            if (k0 + j * BLOCK + threadIdx.x < leaf1) {
-                h[j] = head_out[lr[j].head];
-                m[j] = w.mass[lr[j].mass];
-            }
+        for (uint32_t j = 0; j < LEAF_BATCH; j++) {
+            h[j] = head_out[lr[j].head];
+            m[j] = w.mass[lr[j].mass];
+        }
 #pragma unroll
         for (uint32_t j = 0; j < LEAF_BATCH; j++)
             if (k0 + j * BLOCK + threadIdx.x < leaf1) {
@@ -1244,25 +1292,29 @@ __global__ void k_normalize(WaveDev w, int touched0, int touched1) {
     uint32_t lo = q.lo, hi = q.lo + q.n;
     const bool touched = p ? touched1 : touched0;
     if (q.n <= ROW_BATCH) {  // the row's loads issued together, then the same sum and quotients
-        const float* src = touched ? w.sum : w.cur;
-        float x[ROW_BATCH];
+        const float* src = (touched ? scalar(w.sum) : scalar(w.cur)) + lo;
+        const bool more[ROW_QUADS] = {true, q.n > 4, q.n > 8};
+        float x[ROW_QUADS][4];
 #pragma unroll
-        for (uint32_t k = 0; k < ROW_BATCH; k++)
-            if (k < q.n) x[k] = src[lo + k];
-        if (!touched) {
-#pragma unroll
-            for (uint32_t k = 0; k < ROW_BATCH; k++)
-                if (k < q.n) w.snap[lo + k] = x[k];
-            return;
-        }
+        for (uint32_t h = 0; h < ROW_QUADS; h++)
+            if (more[h]) quad(src + 4 * h, x[h]);
         float s = 0.0f;
 #pragma unroll
-        for (uint32_t k = 0; k < ROW_BATCH; k++)
-            if (k < q.n) s += x[k];
+        for (uint32_t h = 0; h < ROW_QUADS; h++)
+            if (more[h])
+#pragma unroll
+                for (uint32_t k = 0; k < 4; k++) s = 4 * h + k < q.n ? s + x[h][k] : s;
         const float u = 1.0f / (float)(q.n ? q.n : 1);
 #pragma unroll
-        for (uint32_t k = 0; k < ROW_BATCH; k++)
-            if (k < q.n) w.snap[lo + k] = s > 0.0f ? x[k] / s : u;
+        for (uint32_t h = 0; h < ROW_QUADS; h++)
+            if (more[h] && q.n) {
+#pragma unroll
+                for (uint32_t k = 0; k < 4; k++) {
+                    const float y = s > 0.0f ? x[h][k] / s : u;
+                    x[h][k] = touched ? y : x[h][k];
+                }
+                store_quad(w.snap + lo + 4 * h, x[h], q.n - 4 * h);
+            }
         return;
     }
     if (!touched) {
