@@ -54,14 +54,31 @@ struct Blob {
         size = at + std::max<size_t>(bytes, 4);
         return at;
     }
-    void copy_to(uint8_t* dst) const {
-        constexpr size_t CHUNK = size_t(8) << 20;
+    // Copies everything to dst in address order, a segment at a time, calling
+    // sent(offset, bytes) as each is in place: the transfer of one segment
+    // runs while the next is copied (509 MB of tables: 13.5 -> 9.6 ms from
+    // the first copy to the last byte on the device, whose link takes 8.9).
+    template <class F>
+    bool copy_to(uint8_t* dst, F sent) const {
+        constexpr size_t CHUNK = size_t(2) << 20, SEGMENT = size_t(32) << 20;
+        constexpr size_t ALONE = size_t(1) << 20;  // below it, waking helpers takes longer than the copy
         std::vector<Piece> parts;  // pieces cut into chunks of at most CHUNK bytes
         for (const Piece& pc : pieces)
             for (size_t o = 0; o < pc.bytes; o += CHUNK)
                 parts.push_back({pc.src + o, std::min(CHUNK, pc.bytes - o), pc.at + o});
-        parallel_for(
-            parts.size(), [&](size_t k) { std::memcpy(dst + parts[k].at, parts[k].src, parts[k].bytes); }, 8);
+        for (size_t k = 0, at = 0; at < size;) {
+            size_t e = k;
+            while (e < parts.size() && parts[e].at < at + SEGMENT) e++;
+            const size_t end = e < parts.size() ? parts[e].at : size;
+            parallel_for(
+                e - k,
+                [&](size_t i) { std::memcpy(dst + parts[k + i].at, parts[k + i].src, parts[k + i].bytes); },
+                size < ALONE ? 1 : 8);
+            if (!sent(at, end - at)) return false;
+            k = e;
+            at = end;
+        }
+        return true;
     }
 };
 
@@ -500,11 +517,15 @@ bool Executor::upload(const WaveHost& w, const NetBank& bank, uint32_t slot, std
     Slot& sl = slots_[slot];
     if (sl.recorded) HIP_TRY(hipEventSynchronize(sl.uploaded));  // the slot's last upload has left its staging
     if (!ensure_pinned(&sl.pin, &sl.pin_cap, blob.size, err)) return false;
-    blob.copy_to(sl.pin);
     HIP_TRY(hipStreamWaitEvent(copy_, sl.done, 0));  // the slot's last wave no longer reads its tables
-    HIP_TRY(hipMemcpyAsync(table_[slot], sl.pin, blob.size, hipMemcpyHostToDevice, copy_));
-    HIP_TRY(hipEventRecord(sl.uploaded, copy_));  // (recorded again below, after the check)
-    sl.recorded = true;
+    sl.recorded = true;  // (from the first transfer on, the staging may be in use)
+    hipError_t sent = hipSuccess;
+    const bool all = blob.copy_to(sl.pin, [&](size_t at, size_t bytes) {
+        sent = hipMemcpyAsync((char*)table_[slot] + at, sl.pin + at, bytes, hipMemcpyHostToDevice, copy_);
+        if (sent == hipSuccess) sent = hipEventRecord(sl.uploaded, copy_);  // (again below, after the check)
+        return sent == hipSuccess;
+    });
+    if (!all) HIP_TRY(sent);
 
     // Mutable arena.
     const size_t cells = std::max<uint32_t>(w.ncells, 1), rl = std::max<uint32_t>(w.reach_len, 1),
@@ -1241,26 +1262,37 @@ bool Executor::collect(InFlight* f, std::vector<Result>* out, std::string* err) 
     const float* strat = (const float*)sl.res;
     const float* roots = (const float*)(sl.res + f->o_roots);
     const uint16_t* carry = (const uint16_t*)(sl.res + f->o_carry);
-    out->clear();
-    uint32_t cell0 = 0, cfg0 = 0;
-    for (const JobSlice& j : f->jobs) {
-        Result r;
-        r.weight_version = f->version;
-        r.strategy.assign(strat + cell0, strat + cell0 + j.ncells);
-        r.nroots = j.nroots;
-        r.n0 = j.n0;
-        r.n1 = j.n1;
-        r.root_values.assign(roots + j.root_value0, roots + j.root_value0 + j.nroots * (j.n0 + j.n1));
-        r.slots = (uint32_t)f->carry_slots;
-        r.snapshot_configs = j.snapshot_configs;
-        r.carries.resize(size_t(r.slots) * r.snapshot_configs);
-        for (uint32_t s = 0; s < r.slots; s++)
-            std::memcpy(r.carries.data() + size_t(s) * r.snapshot_configs,
-                        carry + size_t(s) * f->snapshot_configs + cfg0, size_t(r.snapshot_configs) * 2);
-        cell0 += j.ncells;
-        cfg0 += r.snapshot_configs;
-        out->push_back(std::move(r));
+    // Each job's share, at offsets from a prefix over the jobs: the copies (and
+    // the first touch of the results' memory) run on several threads when
+    // there is enough of them.
+    const size_t njobs = f->jobs.size();
+    std::vector<size_t> cell0(njobs + 1, 0), cfg0(njobs + 1, 0);
+    for (size_t k = 0; k < njobs; k++) {
+        cell0[k + 1] = cell0[k] + f->jobs[k].ncells;
+        cfg0[k + 1] = cfg0[k] + f->jobs[k].snapshot_configs;
     }
+    out->clear();
+    out->resize(njobs);
+    const size_t bytes = 4 * cell0[njobs] + 2 * f->carry_slots * cfg0[njobs];
+    parallel_for(
+        njobs,
+        [&](size_t k) {
+            const JobSlice& j = f->jobs[k];
+            Result& r = (*out)[k];
+            r.weight_version = f->version;
+            r.strategy.assign(strat + cell0[k], strat + cell0[k + 1]);
+            r.nroots = j.nroots;
+            r.n0 = j.n0;
+            r.n1 = j.n1;
+            r.root_values.assign(roots + j.root_value0, roots + j.root_value0 + j.nroots * (j.n0 + j.n1));
+            r.slots = (uint32_t)f->carry_slots;
+            r.snapshot_configs = j.snapshot_configs;
+            r.carries.resize(size_t(r.slots) * r.snapshot_configs);
+            for (uint32_t s = 0; s < r.slots; s++)
+                std::memcpy(r.carries.data() + size_t(s) * r.snapshot_configs,
+                            carry + size_t(s) * f->snapshot_configs + cfg0[k], size_t(r.snapshot_configs) * 2);
+        },
+        bytes < (size_t(1) << 20) ? 1 : 8);
     return true;
 }
 

@@ -409,7 +409,8 @@ def job_work(b: bytes, precision=WC_PRECISE, route_unit=0, class_shift=0) -> dic
 
 @dataclass
 class SolveResult:
-    """`SolveResult` (engine/src/gpu/client.rs:113-122), copied out of the native result."""
+    """`SolveResult` (engine/src/gpu/client.rs:113-122). strategy and carries are the native result's memory, which
+    lives as long as one of them does; the few root values are a copy, for callers that keep only them."""
     tag: int
     weight_version: int
     strategy: np.ndarray
@@ -422,25 +423,47 @@ class SolveResult:
     @staticmethod
     def take(ptr) -> "SolveResult":
         L = lib()
+        held = _ResultMemory(ptr)
         n = C.c_size_t()
         sp = L.wc_result_strategy(ptr, C.byref(n))
-        strategy = np.ctypeslib.as_array(sp, (n.value,)).copy() if n.value else np.zeros(0, np.float32)
+        strategy = held.array(sp, n.value, "<f4")
         nr, n0, n1 = C.c_uint32(), C.c_uint32(), C.c_uint32()
         rp = L.wc_result_root_values(ptr, C.byref(nr), C.byref(n0), C.byref(n1))
-        k = nr.value * (n0.value + n1.value)
-        roots = (np.ctypeslib.as_array(rp, (k,)).copy() if k else np.zeros(0, np.float32)).reshape(
-            nr.value, n0.value + n1.value)
+        roots = held.array(rp, nr.value * (n0.value + n1.value), "<f4").copy().reshape(nr.value,
+                                                                                            n0.value + n1.value)
         slots, cfgs = C.c_uint32(), C.c_uint32()
         cp = L.wc_result_carries(ptr, C.byref(slots), C.byref(cfgs))
-        k = slots.value * cfgs.value
-        carries = (np.ctypeslib.as_array(cp, (k,)).copy() if k else np.zeros(0, np.uint16)).view(
-            np.float16).reshape(slots.value, cfgs.value)
+        carries = held.array(cp, slots.value * cfgs.value, "<f2").reshape(slots.value, cfgs.value)
         ov, card = C.c_int(), C.c_int()
         _check(L.wc_result_routes(ptr, C.byref(ov), C.byref(card)))
-        r = SolveResult(int(L.wc_result_tag(ptr)), int(L.wc_result_weight_version(ptr)), strategy, roots,
-                        (n0.value, n1.value), carries, bool(ov.value), bool(card.value))
-        L.wc_result_free(ptr)
-        return r
+        return SolveResult(int(L.wc_result_tag(ptr)), int(L.wc_result_weight_version(ptr)), strategy, roots,
+                           (n0.value, n1.value), carries, bool(ov.value), bool(card.value))
+
+
+class _ResultMemory:
+    """A native result, freed when the last array over its memory is gone."""
+
+    class View:
+        """One of its arrays, for numpy's array interface."""
+
+        def __init__(self, owner, address, count, typestr):
+            self.owner = owner
+            self.__array_interface__ = {"data": (address, False), "shape": (count,), "typestr": typestr, "version": 3}
+
+    def __init__(self, ptr):
+        self.ptr = ptr
+
+    def array(self, at, count, typestr):
+        """The result's memory at a pointer as an array (no copy) that keeps it alive."""
+        if not count:
+            return np.zeros(0, np.dtype(typestr))
+        return np.asarray(_ResultMemory.View(self, C.cast(at, C.c_void_p).value, count, typestr))
+
+    def __del__(self):
+        try:
+            lib().wc_result_free(self.ptr)
+        except Exception:
+            pass
 
 
 # ------------------------------------------------------------------ executor
