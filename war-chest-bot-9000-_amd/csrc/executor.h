@@ -175,8 +175,11 @@ class Executor {
     bool launch_wave(const WaveHost& w, uint64_t version, InFlight* out, std::string* err,
                      std::function<void()>* meanwhile);
     // `meanwhile` (if set) is called and cleared while a device check runs.
+    // build_early: the schedule follows at once, so the v5 network's per-wave
+    // build may be queued while the rest of the tables is on its way (built_);
+    // a wave still to be checked on the device waits for its check.
     bool upload(const WaveHost& w, const NetBank& bank, uint32_t slot, std::string* err, bool device_check = false,
-                std::function<void()>* meanwhile = nullptr);
+                std::function<void()>* meanwhile = nullptr, bool build_early = false);
     // The device element checks of the uploaded wave; waits for their result.
     bool check_on_device(const WaveHost& w, std::string* err, std::function<void()>* meanwhile);
     // hook (optional): called after every leaf-net evaluation with its
@@ -269,6 +272,7 @@ class Executor {
     const uint32_t* top_reach_chunk_dev_[2] = {};  // chunk bounds of the fused reach launches
     const uint32_t* top_reach_par_dev_[2] = {};    // and the shallower rows each chunk computes
     const uint32_t* head_tile_n_ = nullptr;  // head width per 128-row tile (device copy)
+    bool built_ = false;  // the uploaded wave's v5 build is queued already; the next schedule leaves it out
     const uint32_t* head_rb_n_[2] = {};      // head width per 16-row block and traverser (device copies)
     const ChainPass* chain_plan_[2] = {};    // fused value net passes per traverser (device copies)
     uint32_t chain_npass_[2] = {0, 0};
