@@ -12,6 +12,7 @@ import pytest
 
 import oracle as O
 import warchest_wave as ww
+import workloads as W
 from test_zz_no_alloc import Hip
 
 pytestmark = pytest.mark.gpu
@@ -109,3 +110,27 @@ def test_compensated_fused_net(inputs, hidden, layers, heads, rows, offset):
         h, at, k = np.maximum(h @ w + net.b[layer * hidden:(layer + 1) * hidden], 0.0), at + k * hidden, hidden
     ref = h @ net.w[at:].reshape(heads, hidden).T.astype(np.float64) + net.b[layers * hidden:]
     assert np.abs(got[:500] - ref).max() <= 1e-5 * np.abs(ref).max()
+
+
+# idle wavefronts, one to four feature blocks each, one to three layers; few rows and several blocks per pass
+@pytest.mark.parametrize("precision,mode,bound", [(ww.WC_F16, O.NET_F16, 2e-3), (ww.WC_BF16, O.NET_BF16, 1e-2)])
+@pytest.mark.parametrize("inputs,width,layers,trees,nodes", [
+    (160, 32, 1, 1, 12), (192, 96, 2, 2, 60), (512, 288, 3, 3, 90), (256, 512, 2, 12, 400), (512, 416, 1, 40, 400)])
+def test_fused_public_tower(precision, mode, bound, inputs, width, layers, trees, nodes):
+    """The wave's leaf values at the initial reach against the oracle's model of the operand rounding, within the
+    bounds of the full waves' leaf probes."""
+    say(f"case fused tower {precision}: {inputs} -> {layers}x{width}, {trees} trees of {nodes} nodes")
+    dims = ww.two_tower_dims(inputs=inputs, width=width, pub_layers=layers, priv_in=32, priv_layers=1, pool=64)
+    jobs = ww.synth_jobs(dims, seed=width, trees=trees, nodes_lo=nodes, nodes_hi=nodes + 9, act_lo=3, act_hi=8,
+                         collapse=0.6, chance=1, draw_lo=2, draw_hi=3, info_fixed=9, dirichlet=1, iters=2, depth=2,
+                         snapshots=1, nroots=1, **W.DCFR)
+    net = ww.synth_weights(dims, seed=layers)
+    ex = ww.Executor(0, precision)
+    wave = ww.Wave(jobs)
+    got, _ = ex.leaf_probe(wave, ex.publish(net), 0)
+    rows = wave.stats()["rows"]
+    wave.close()
+    ex.close()
+    want = np.concatenate([O.leaf_probe(j, net, mode, 0)[0] for j in jobs])
+    say(f"  {rows} rows, max error {np.abs(got - want).max() / np.abs(want).max():.1e} of the largest value")
+    assert np.abs(got - want).max() <= bound * np.abs(want).max()

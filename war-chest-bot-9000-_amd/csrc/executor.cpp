@@ -853,6 +853,11 @@ void Executor::run_tower_private(const NetBank& bank) {
 void Executor::run_tower(const NetBank& bank, uint32_t rows, int traverser) {
     const NetShape& ns = bank.ns;
     const void* in = Xq_[traverser];
+    if (precision_ != WC_PRECISE && tower_fits(ns.in, ns.hidden, ns.layers)) {
+        launch_tower(precision_, chain_net(bank), in, H_[0], rows, cus_, stream_);
+        launch_tower_head(dev_, traverser, precision_, H_[0], ns.hidden, F_, bank.bread, head_out_, stream_);
+        return;
+    }
     uint32_t k = ns.in;
     for (uint32_t l = 0; l < ns.layers; l++) {
         void* out = H_[l & 1];

@@ -200,6 +200,12 @@ void launch_chain_rows(int precision, ChainNet net, const float* X, uint32_t row
 // row block of the plan.
 void launch_chain_static(int precision, const ChainNet& net, const void* X, float* part, const ChainPass* plan,
                          uint32_t npass, hipStream_t s);
+// The public tower in one launch (16-bit operands; `cus` compute units to deal
+// its passes over): X and Y fragment-major with gemm_rows(rows) rows, net's
+// trunk layers. Applies when tower_fits(in, width, layers).
+bool tower_fits(uint32_t in, uint32_t width, uint32_t layers);
+void launch_tower(int precision, const ChainNet& net, const void* X, void* Y, uint32_t rows, uint32_t cus,
+                  hipStream_t s);
 // Two-tower net: F = private-tower output (ncfg rows, fragment-major 16-bit or
 // row-major f32) times the readout weight, row-major; then player p's readout
 // blocks, tv[entry (row, config)] = <F[config], H[row]> + bread, from the

@@ -2352,6 +2352,164 @@ __global__ __launch_bounds__(CHAIN_WAVES * 64) __attribute__((amdgpu_waves_per_e
     }
 }
 
+// ------------------------------------------------ fused public tower
+//
+// The two-tower net's public tower, up to TOWER_WIDTH wide, in one launch: a
+// pass of up to four 16-row blocks staged in LDS, every layer in place as in
+// k_chain (each wavefront owns up to four 16-feature blocks of the width), the
+// last layer stored as the readout's fragment-major operand. k_gemm's products
+// in k_gemm's order: bit-identical. Bound: each pass streams the weights from
+// L2 (1 MB for 512 -> 2x512) and 188 registers leave one workgroup per CU;
+// layer by layer every activation crossed HBM twice and a 128-wide tile filled
+// 280 workgroups. 8,904 rows: 50 -> 27 us per pass; 49 row blocks (784 rows):
+// 28 -> 10 us.
+
+constexpr int TOWER_RB = 4, TOWER_NB = 4;
+constexpr uint32_t TOWER_WIDTH = CHAIN_WAVES * TOWER_NB * 16;
+
+bool tower_fits(uint32_t in, uint32_t width, uint32_t layers) {
+    return in % 32 == 0 && in <= TOWER_WIDTH && width % 32 == 0 && width <= TOWER_WIDTH && layers >= 1 &&
+           layers <= CHAIN_MAX_LAYERS;
+}
+
+template <int PREC, int NB, int RB>
+__device__ __forceinline__ void tower_kloop(float4v (&acc)[TOWER_RB][TOWER_NB], const uint16_t* xs, uint32_t ks,
+                                            const uint16_t* __restrict__ wp, size_t wstride) {
+#pragma unroll
+    for (int a = 0; a < RB; a++)
+#pragma unroll
+        for (int b = 0; b < NB; b++) acc[a][b] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
+    uint4 xa[RB], xb[RB], w0[NB], w1[NB], w2[NB], w3[NB];
+    auto ldw = [&](uint4 (&fw)[NB], uint32_t s) {
+        s = s < ks ? s : ks - 1;
+#pragma unroll
+        for (int b = 0; b < NB; b++) fw[b] = *(const uint4*)(wp + b * wstride + (size_t)s * 512);
+    };
+    auto ldx = [&](uint4 (&fx)[RB], uint32_t s) {
+        s = s < ks ? s : ks - 1;
+#pragma unroll
+        for (int a = 0; a < RB; a++) fx[a] = *(const uint4*)(xs + ((size_t)a * ks + s) * 512);
+    };
+    auto step = [&](const uint4 (&fx)[RB], const uint4 (&fw)[NB]) {
+#pragma unroll
+        for (int a = 0; a < RB; a++)
+#pragma unroll
+            for (int b = 0; b < NB; b++) acc[a][b] = mfma16<PREC>(fw[b], fx[a], acc[a][b]);
+    };
+    ldw(w0, 0);
+    ldw(w1, 1);
+    ldx(xa, 0);
+    uint32_t s = 0;
+    for (; s + 4 <= ks; s += 4) {
+        ldw(w2, s + 2);
+        ldx(xb, s + 1);
+        __builtin_amdgcn_sched_barrier(0);
+        step(xa, w0);
+        __builtin_amdgcn_sched_barrier(0);
+        ldw(w3, s + 3);
+        ldx(xa, s + 2);
+        __builtin_amdgcn_sched_barrier(0);
+        step(xb, w1);
+        __builtin_amdgcn_sched_barrier(0);
+        ldw(w0, s + 4);
+        ldx(xb, s + 3);
+        __builtin_amdgcn_sched_barrier(0);
+        step(xa, w2);
+        __builtin_amdgcn_sched_barrier(0);
+        ldw(w1, s + 5);
+        ldx(xa, s + 4);
+        __builtin_amdgcn_sched_barrier(0);
+        step(xb, w3);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    for (; s < ks; s++) {  // K not a multiple of 128: the last steps one at a time
+        ldw(w0, s);
+        ldx(xa, s);
+        step(xa, w0);
+    }
+}
+
+template <int PREC, int RB>
+__device__ __forceinline__ void tower_pass(const ChainNet& net, const uint16_t* __restrict__ X,
+                                           uint16_t* __restrict__ Y, uint32_t rb0, uint16_t* lds, uint32_t lane,
+                                           uint32_t wave) {
+    const uint32_t q = lane >> 4, r = lane & 15;
+    const uint32_t hblk = net.hidden >> 4, ksn = net.hidden >> 5, ks0 = net.in >> 5;
+    const uint32_t nb = hblk > wave ? (hblk - wave + CHAIN_WAVES - 1) / CHAIN_WAVES : 0;
+    // consecutive blocks: one contiguous run
+    const uint4* src = (const uint4*)(X + (size_t)rb0 * ks0 * 512);
+    for (uint32_t i = threadIdx.x; i < RB * ks0 * 64; i += CHAIN_WAVES * 64) ((uint4*)lds)[i] = src[i];
+    float4v acc[TOWER_RB][TOWER_NB];
+    __syncthreads();
+    for (uint32_t l = 0; l < net.layers; l++) {
+        const uint32_t ks = l ? ksn : ks0;
+        const uint16_t* xs = lds + lane * 8;
+        const uint16_t* wp = net.w[l] + ((size_t)wave * ks * 64 + lane) * 8;
+        const size_t wstride = (size_t)CHAIN_WAVES * ks * 512;
+        static_assert(TOWER_NB == 4, "dispatch below covers 1..4 blocks");
+        if (nb == 1)
+            tower_kloop<PREC, 1, RB>(acc, xs, ks, wp, wstride);
+        else if (nb == 2)
+            tower_kloop<PREC, 2, RB>(acc, xs, ks, wp, wstride);
+        else if (nb == 3)
+            tower_kloop<PREC, 3, RB>(acc, xs, ks, wp, wstride);
+        else if (nb == 4)
+            tower_kloop<PREC, 4, RB>(acc, xs, ks, wp, wstride);
+        __syncthreads();  // the layer input is dead from here on
+        const float* bias = net.b[l];
+#pragma unroll
+        for (int b = 0; b < TOWER_NB; b++) {
+            if ((uint32_t)b >= nb) break;
+            const uint32_t n = (wave + CHAIN_WAVES * b) * 16 + 4 * q;
+            float bv[4];
+#pragma unroll
+            for (int v = 0; v < 4; v++) bv[v] = bias[n + v];
+            const size_t col = (size_t)(n >> 5) * 64 + r + ((n & 31) >> 3) * 16;
+#pragma unroll
+            for (int a = 0; a < RB; a++) {
+                uint16_t h[4];
+#pragma unroll
+                for (int v = 0; v < 4; v++) {
+                    const float y = acc[a][b][v] + bv[v];
+                    h[v] = PREC == WC_F16 ? f32_to_f16_rn(y > 0.0f ? y : 0.0f) : f32_to_bf16_rn(y > 0.0f ? y : 0.0f);
+                }
+                *(uint2*)(lds + (((size_t)a * ksn * 64 + col) * 8 + (n & 7))) =
+                    make_uint2(pack16(h[0], h[1]), pack16(h[2], h[3]));
+            }
+        }
+        __syncthreads();
+    }
+    uint4* dst = (uint4*)(Y + (size_t)rb0 * ksn * 512);
+    for (uint32_t i = threadIdx.x; i < RB * ksn * 64; i += CHAIN_WAVES * 64) dst[i] = ((const uint4*)lds)[i];
+}
+
+// One workgroup per pass of `per` consecutive row blocks of nrb.
+template <int PREC>
+__global__ __launch_bounds__(CHAIN_WAVES * 64) void k_tower(ChainNet net, const uint16_t* __restrict__ X,
+                                                            uint16_t* __restrict__ Y, uint32_t nrb, uint32_t per) {
+    __shared__ __attribute__((aligned(16))) uint16_t lds[TOWER_RB * 16 * TOWER_WIDTH];
+    const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6, rb0 = blockIdx.x * per;
+    switch (min(per, nrb - rb0)) {
+        case 4: tower_pass<PREC, 4>(net, X, Y, rb0, lds, lane, wave); break;
+        case 3: tower_pass<PREC, 3>(net, X, Y, rb0, lds, lane, wave); break;
+        case 2: tower_pass<PREC, 2>(net, X, Y, rb0, lds, lane, wave); break;
+        case 1: tower_pass<PREC, 1>(net, X, Y, rb0, lds, lane, wave); break;
+        default: break;
+    }
+}
+
+void launch_tower(int precision, const ChainNet& net, const void* X, void* Y, uint32_t rows, uint32_t cus,
+                  hipStream_t s) {
+    if (!rows) return;
+    const uint32_t nrb = (rows + 15) / 16, rounds = (nrb + TOWER_RB * cus - 1) / (TOWER_RB * cus);
+    const uint32_t per = (nrb + rounds * cus - 1) / (rounds * cus);  // (one workgroup's registers fill a CU)
+    const dim3 grid((nrb + per - 1) / per), block(CHAIN_WAVES * 64);
+    if (precision == WC_F16)
+        hipLaunchKernelGGL(k_tower<WC_F16>, grid, block, 0, s, net, (const uint16_t*)X, (uint16_t*)Y, nrb, per);
+    else
+        hipLaunchKernelGGL(k_tower<WC_BF16>, grid, block, 0, s, net, (const uint16_t*)X, (uint16_t*)Y, nrb, per);
+}
+
 void launch_chain(int precision, const ChainNet& net, const void* X, uint32_t rows, float* out,
                   const ChainPass* plan, uint32_t npass, hipStream_t s) {
     if (rows == 0 || npass == 0) return;
