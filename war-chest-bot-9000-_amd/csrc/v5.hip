@@ -680,6 +680,7 @@ constexpr int JT_ROWS = 32;          // rows per join workgroup
 constexpr int JT_WAVES = 8;          // wavefront w owns columns 16 w .. 16 w + 15 of the 128-wide stream
 constexpr int JT_LD = JW + 8;        // LDS row stride of the 16-bit operand (halves)
 constexpr int JT_RB = JT_ROWS / 16;  // row blocks per tile
+constexpr int JT_HLD = D + 8;        // LDS row stride of the output tile (halves)
 
 // Net::join for a 64-row tile on the matrix cores (16x16x32, 16-bit operands,
 // f32 accumulate). Eight wavefronts: wavefront w owns one 16-column block of
@@ -690,13 +691,21 @@ constexpr int JT_RB = JT_ROWS / 16;  // row blocks per tile
 // k steps) are loaded before the norm that precedes the product, so their L2
 // latency overlaps it. In the accumulator layout lane l holds rows
 // 4 (l / 16) + v, column l % 16 of each 16 x 16 tile; an A fragment is 8
-// consecutive k of row l % 16.
+// consecutive k of row l % 16. Bound: the VALU of the norms and GELUs and the
+// barriers between wavefronts that share rows, two per norm: 49,371 rows take 63
+// us, 193 rows 11.5 (70 and 14 with four barriers per norm, one wavefront
+// combining the statistics and 2-byte output stores).
 template <int PREC>
 __global__ __launch_bounds__(JT_WAVES * 64) void k_join_mfma(Net net, uint32_t rows, const uint16_t* __restrict__ X,
                                                             const float* __restrict__ P, const float* __restrict__ Jp,
                                                             uint16_t* __restrict__ H) {
-    __shared__ __attribute__((aligned(16))) uint16_t tA[JT_ROWS * JT_LD];
-    __shared__ float part[JT_WAVES][JT_ROWS], part2[JT_WAVES][JT_ROWS], mean[JT_ROWS], inv[JT_ROWS];
+    // The operand twice, so that the next norm may write one while a slower
+    // wavefront still reads the other; the output tile takes both at the end.
+    __shared__ __attribute__((aligned(16))) uint16_t tA[2][JT_ROWS * JT_LD];
+    __shared__ float part[JT_WAVES][JT_ROWS], part2[JT_WAVES][JT_ROWS];
+    __shared__ __attribute__((aligned(16))) float stat[JT_WAVES][2][JT_ROWS];  // each wavefront's own copy
+    static_assert(sizeof tA >= JT_ROWS * JT_HLD * sizeof(uint16_t), "the output tile fits the operands");
+    int buf = 0;
     const uint32_t wv = threadIdx.x >> 6, l = threadIdx.x & 63, q = l >> 4, i = l & 15;
     const uint32_t r0 = blockIdx.x * JT_ROWS;
     const uint32_t col = wv * 16 + i;  // this lane's column of the 128-wide stream
@@ -705,6 +714,9 @@ __global__ __launch_bounds__(JT_WAVES * 64) void k_join_mfma(Net net, uint32_t r
     // Each wavefront's sum and sum of squared deviations from its own mean
     // (over its NC x 16 columns), combined across the wavefronts by the
     // pairwise-variance formula (Chan, Golub and LeVeque) in one exchange.
+    // Every wavefront combines all rows itself, lane r row r, and reads its
+    // lanes' rows back from its own copy: one barrier.
+    float mean[JT_RB][4], inv[JT_RB][4];  // of rows rb * 16 + 4 q + v
     auto row_stats = [&](auto& z, auto ncb, float width) {
         constexpr uint32_t NC = decltype(ncb)::value;
         constexpr float NW = 16.0f * NC;  // columns per wavefront
@@ -742,21 +754,30 @@ __global__ __launch_bounds__(JT_WAVES * 64) void k_join_mfma(Net net, uint32_t r
                     part2[wv][rb * 16 + 4 * q + v] = dw[rb * 4 + v];
                 }
         __syncthreads();
-        if (threadIdx.x < JT_ROWS) {
+        {
+            const uint32_t r = l % JT_ROWS;
             float t = 0.0f;
 #pragma unroll
-            for (uint32_t w2 = 0; w2 < JT_WAVES; w2++) t += part[w2][threadIdx.x];
+            for (uint32_t w2 = 0; w2 < JT_WAVES; w2++) t += part[w2][r];
             const float m = t / width;
             float m2 = 0.0f;
 #pragma unroll
             for (uint32_t w2 = 0; w2 < JT_WAVES; w2++) {
-                const float dm = part[w2][threadIdx.x] * (1.0f / NW) - m;
-                m2 += part2[w2][threadIdx.x] + NW * dm * dm;
+                const float dm = part[w2][r] * (1.0f / NW) - m;
+                m2 += part2[w2][r] + NW * dm * dm;
             }
-            mean[threadIdx.x] = m;
-            inv[threadIdx.x] = 1.0f / sqrtf(m2 / width + 1e-5f);
+            stat[wv][0][r] = m;
+            stat[wv][1][r] = 1.0f / sqrtf(m2 / width + 1e-5f);
         }
-        __syncthreads();
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+        for (uint32_t rb = 0; rb < JT_RB; rb++)
+#pragma unroll
+            for (uint32_t v = 0; v < 4; v++) {
+                mean[rb][v] = stat[wv][0][rb * 16 + 4 * q + v];
+                inv[rb][v] = stat[wv][1][rb * 16 + 4 * q + v];
+            }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     };
     // gelu(LN(z)) of the 128-wide stream into the A operand in LDS (16-bit).
     auto to_operand = [&](float (&z)[JT_RB][1][4], uint32_t which) {
@@ -767,7 +788,7 @@ __global__ __launch_bounds__(JT_WAVES * 64) void k_join_mfma(Net net, uint32_t r
 #pragma unroll
             for (uint32_t v = 0; v < 4; v++) {
                 const uint32_t r = rb * 16 + 4 * q + v;
-                tA[r * JT_LD + col] = to16<PREC>(gelu_fast((z[rb][0][v] - mean[r]) * inv[r] * g + bt));
+                tA[buf][r * JT_LD + col] = to16<PREC>(gelu_fast((z[rb][0][v] - mean[rb][v]) * inv[rb][v] * g + bt));
             }
         __syncthreads();
     };
@@ -795,7 +816,7 @@ __global__ __launch_bounds__(JT_WAVES * 64) void k_join_mfma(Net net, uint32_t r
 #pragma unroll
             for (uint32_t rb = 0; rb < JT_RB; rb++)
                 af[rb] = from_x ? *(const uint4*)(X + ((size_t)((r0 >> 4) + rb) * KS * 64 + (size_t)s * 64 + l) * 8)
-                                : *(const uint4*)(tA + (rb * 16 + i) * JT_LD + s * 32 + 8 * q);
+                                : *(const uint4*)(tA[buf] + (rb * 16 + i) * JT_LD + s * 32 + 8 * q);
 #pragma unroll
             for (uint32_t rb = 0; rb < JT_RB; rb++)
 #pragma unroll
@@ -815,9 +836,9 @@ __global__ __launch_bounds__(JT_WAVES * 64) void k_join_mfma(Net net, uint32_t r
         for (uint32_t rb = 0; rb < JT_RB; rb++)
 #pragma unroll
             for (uint32_t v = 0; v < 4; v++) {
-                const uint32_t row = r0 + rb * 16 + 4 * q + v;
-                const float jp = row < rows ? Jp[(size_t)row * JW + col] : 0.0f;
-                z[rb][0][v] = (jp + acc[rb][0][v]) + bias;
+                // (a row past the last repeats it: its outputs are not stored)
+                const uint32_t row = min(r0 + rb * 16 + 4 * q + v, rows - 1);
+                z[rb][0][v] = (Jp[(size_t)row * JW + col] + acc[rb][0][v]) + bias;
             }
     }
     for (uint32_t blk = 0; blk < JBLOCKS; blk++) {
@@ -825,7 +846,7 @@ __global__ __launch_bounds__(JT_WAVES * 64) void k_join_mfma(Net net, uint32_t r
         to_operand(z, LN_JOIN + blk);
         v5f4 acc[JT_RB][1];
         gemm(acc, bw, false);
-        __syncthreads();  // every wave has read the operand before the next one is written
+        buf ^= 1;
         const float bias = net.b[LY.join_w[blk].b + col];
 #pragma unroll
         for (uint32_t rb = 0; rb < JT_RB; rb++)
@@ -847,9 +868,8 @@ __global__ __launch_bounds__(JT_WAVES * 64) void k_join_mfma(Net net, uint32_t r
             const float bias = net.b[LY.join_out.b + c2];
 #pragma unroll
             for (uint32_t v = 0; v < 4; v++) {
-                const uint32_t row = r0 + rb * 16 + 4 * q + v;
-                const float pv = row < rows ? P[(size_t)row * D + c2] : 0.0f;
-                h[rb][cb][v] = (pv + acc[rb][cb][v]) + bias;
+                const uint32_t row = min(r0 + rb * 16 + 4 * q + v, rows - 1);
+                h[rb][cb][v] = (P[(size_t)row * D + c2] + acc[rb][cb][v]) + bias;
             }
         }
     row_stats(h, std::integral_constant<uint32_t, 2>{}, (float)D);
@@ -861,9 +881,16 @@ __global__ __launch_bounds__(JT_WAVES * 64) void k_join_mfma(Net net, uint32_t r
         for (uint32_t rb = 0; rb < JT_RB; rb++)
 #pragma unroll
             for (uint32_t v = 0; v < 4; v++) {
-                const uint32_t r = rb * 16 + 4 * q + v, row = r0 + r;
-                if (row < rows) H[frag_off(row, c2, D)] = to16<PREC>((h[rb][cb][v] - mean[r]) * inv[r] * g + bt);
+                const uint32_t r = rb * 16 + 4 * q + v;
+                tA[0][r * JT_HLD + c2] = to16<PREC>((h[rb][cb][v] - mean[rb][v]) * inv[rb][v] * g + bt);
             }
+    }
+    __syncthreads();
+    // The tile as fragments, one 16-byte run per lane, in the order they are stored.
+    for (uint32_t e = threadIdx.x; e < JT_RB * (D / 32) * 64; e += JT_WAVES * 64) {
+        const uint32_t rb = e / (D / 32 * 64), s = e / 64 % (D / 32), row = rb * 16 + e % 16, k = 32 * s + e % 64 / 16 * 8;
+        if (r0 + row < rows)
+            *(uint4*)(H + frag_off(r0 + row, k, D)) = *(const uint4*)(tA[0] + row * JT_HLD + k);
     }
 }
 
