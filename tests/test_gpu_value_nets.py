@@ -39,10 +39,11 @@ def forward_on_device(ex, v, x, heads, offset):
         hip.free(od)
 
 
-# rows x outputs cross the line between the 16-, 32- and 64-wide tiles
+# rows x outputs cross the lines between the four tile sizes
 @pytest.mark.parametrize("inputs,hidden,layers,heads,rows,offset", [
     (101, 50, 2, 7, 1, 0), (130, 64, 1, 1, 17, 1), (512, 384, 3, 22, 64, 0), (97, 130, 2, 567, 333, 3),
-    (160, 384, 2, 33, 1500, 2), (132, 384, 1, 65, 5500, 0), (31, 391, 1, 22, 6001, 1)])
+    (160, 384, 2, 33, 1500, 2), (132, 384, 1, 567, 3100, 1),
+    (132, 384, 1, 65, 5500, 0), (31, 391, 1, 22, 6001, 1)])
 def test_float32_net_edges(inputs, hidden, layers, heads, rows, offset):
     say(f"case float32 net: {rows} rows, {inputs} -> {layers}x{hidden} -> {heads}, buffers + {offset} floats")
     net = ww.synth_weights(ww.mlp_dims(inputs, hidden, layers, heads, pool=8), seed=rows)

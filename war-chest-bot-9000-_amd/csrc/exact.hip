@@ -10,9 +10,9 @@
 //
 // Bound: two VALU operations per product (about 19.7e12 products per second
 // over 256 CUs without packed or fused arithmetic). A 384 -> 384 layer of 3,915
-// rows takes 41 us (15.6e12 products per second over a wave's three layers)
+// rows takes 41 us (15.6e12 products per second over a wave's three layers; 37 us with 64 x 32 tiles)
 // against 319 us with one output per thread and its operands read through L1;
-// the whole 512 -> 3x384 -> 567 net of 3,001 rows 144 us against 3,290.
+// the whole 512 -> 3x384 -> 567 net of 3,001 rows 142 us against 3,290.
 #include "kernels.h"
 
 #include <algorithm>
@@ -23,9 +23,11 @@ namespace {
 
 constexpr uint32_t THREADS = 256, SIDE = 16;  // a SIDE x SIDE grid of threads over the tile
 // A larger tile reads less LDS per product but needs enough workgroups: the
-// largest one with at least two per CU is taken. 3,001 rows (282 tiles of 64
-// for a 384-wide layer): 144 us with 32-wide tiles, 171 us with 64-wide ones;
-// 8,000 rows (750 tiles): 205 us with 64-wide tiles, 231 us with 32-wide.
+// largest one with at least two per CU is taken. 3,001 rows (282 tiles of 64 x
+// 64 for a 384-wide layer, 564 of 64 x 32): 142 us with 64 x 32 tiles, 148 with
+// 32 x 32, 171 with 64 x 64; 8,000 rows (750 of 64 x 64): 206 us with 64 x 64
+// tiles, 231 with 32 x 32. The smallest tile's k tile: 60 rows take 28.6 us
+// with 128 inputs, 30.6 with 32, 33.5 with 256.
 constexpr uint64_t MIN_TILES = 512;
 
 enum : uint32_t { VEC_X = 1, VEC_W = 2 };  // 16-byte loads of the operand are aligned
@@ -181,12 +183,16 @@ void launch(bool head, bool skip, const float* X, uint32_t K, const float* Wt, c
 void dispatch(bool head, bool skip, const float* X, uint32_t K, const float* Wt, const float* b, uint32_t N, float* Y,
               uint32_t M, const uint32_t* rb_n, hipStream_t s) {
     if (!M || !N) return;
-    auto tiles = [&](uint32_t side) { return (uint64_t)((M + side - 1) / side) * ((N + side - 1) / side); };
+    auto tiles = [&](uint32_t rows, uint32_t cols) {
+        return (uint64_t)((M + rows - 1) / rows) * ((N + cols - 1) / cols);
+    };
     // With per-block column bounds a finer tile also skips more columns (the
     // 64-subgame wave: 38 us per head with 64-wide tiles, about 20 with 32).
-    if (tiles(64) >= MIN_TILES && !rb_n)
+    if (tiles(64, 64) >= MIN_TILES && !rb_n)
         launch<4, 4, 32>(head, skip, X, K, Wt, b, N, Y, M, rb_n, s);
-    else if (tiles(32) >= MIN_TILES)
+    else if (tiles(64, 32) >= MIN_TILES && !rb_n)
+        launch<4, 2, 32>(head, skip, X, K, Wt, b, N, Y, M, rb_n, s);
+    else if (tiles(32, 32) >= MIN_TILES)
         launch<2, 2, 64>(head, skip, X, K, Wt, b, N, Y, M, rb_n, s);
     else
         launch<1, 1, 128>(head, skip, X, K, Wt, b, N, Y, M, rb_n, s);
