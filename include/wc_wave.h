@@ -31,8 +31,7 @@ extern "C" {
  * fast mode, CUBLAS_COMPUTE_32F_FAST_16F). F16X (no counterpart in the
  * reference) is compensated f16: every operand is held as an f16 pair
  * hi + lo and every product as three f16 MFMAs (hi hi + hi lo + lo hi) with
- * f32 accumulation, near float32 accuracy on the f16 matrix cores; MLP only,
- * layer by layer. */
+ * f32 accumulation, near float32 accuracy on the f16 matrix cores; MLP only. */
 #define WC_PRECISE 0
 #define WC_F16 1
 #define WC_BF16 2
@@ -329,10 +328,10 @@ int wc_mlp_forward(wc_executor* ex, uint64_t version, uint32_t rows, const float
 /* No counterpart in the reference: for callers that cannot allocate device
  * memory (code under HIP graph capture, tight serving loops, harnesses that
  * forbid hipMalloc). wc_mlp_forward on device-resident buffers -- x: rows x in
- * f32, out: rows x heads f32 -- with every intermediate (the 16-bit input
- * operand, hidden activations, the pass plan) in one fixed device array of
- * WC_NOALLOC_SCRATCH_BYTES per GPU, held until the process ends; the call
- * makes no device allocation. stream NULL: queued on the executor's stream
+ * f32, out: rows x heads f32 -- with every intermediate it needs (a
+ * layer-by-layer net's input operand and hidden activations) in one fixed
+ * device array of WC_NOALLOC_SCRATCH_BYTES per GPU, held until the process
+ * ends; the call makes no device allocation. stream NULL: queued on the executor's stream
  * and the call waits for the result; otherwise queued on that hipStream_t and
  * the call returns at once. Calls that overlap on one GPU share the array and
  * race. Fails (WC_ERR_INVALID) when the rows need more than the array holds

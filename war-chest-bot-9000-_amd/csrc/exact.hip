@@ -10,9 +10,10 @@
 //
 // Bound: two VALU operations per product (about 19.7e12 products per second
 // over 256 CUs without packed or fused arithmetic). A 384 -> 384 layer of 3,915
-// rows takes 41 us (15.6e12 products per second over a wave's three layers; 37 us with 64 x 32 tiles)
-// against 319 us with one output per thread and its operands read through L1;
-// the whole 512 -> 3x384 -> 567 net of 3,001 rows 142 us against 3,290.
+// rows takes 38 us with 64 x 32 tiles (16.9e12 products per second over a wave's
+// three layers), 41 us with 32 x 32 and 319 us with one output per thread and
+// its operands read through L1; the whole 512 -> 3x384 -> 567 net of 3,001 rows
+// 142 us against 3,290.
 #include "kernels.h"
 
 #include <algorithm>

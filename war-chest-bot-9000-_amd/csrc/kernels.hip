@@ -491,8 +491,8 @@ __device__ __forceinline__ float lane_sum_in_order(float tot, float v, uint32_t 
 // five more scalar instructions) and a lane read, a product and a sum, with 16
 // configs' loads in flight ahead of them: 64 depth-1 subgames 52 -> 32 us per
 // launch, 32 depth-2 subgames 48 -> 30 us. WIDE: a table of 4 GiB or more.
-// The pooled block goes straight into the two query inputs that carry it: [pooled_q | pooled_{1-q} | seat | public] for
-// traverser q.
+// The pooled block goes straight into the two query inputs that carry it:
+// [pooled_q | pooled_{1-q} | seat | public] for traverser q.
 template <bool WIDE>
 __global__ __launch_bounds__(BLOCK) void k_pool_exact(WaveDev w, int player, float* x0, float* x1, int acc,
                                                     float ds, uint32_t pool_blocks) {
