@@ -1005,7 +1005,7 @@ __device__ __forceinline__ void backprop_row(const WaveDev& w, int p, BackRec q,
     // predict delta, EPS), normalised by a reciprocal multiply. The sum's
     // discount (sum *= ds) is taken with the accumulation in the reach sweep.
     const float* st = MODE == MODE_VALUE ? strat : w.cur;
-    if (n <= ROW_BATCH) {  // everything stays in registers
+    if (n - 1 < ROW_BATCH) {  // 1 to 12 actions: everything stays in registers
         uint32_t lvi[ROW_QUADS][4];
         float sv[ROW_QUADS][4], qv[ROW_QUADS][4], old[ROW_QUADS][4];
         const bool more[ROW_QUADS] = {true, n > 4, n > 8};
@@ -1064,7 +1064,8 @@ __device__ __forceinline__ void backprop_row(const WaveDev& w, int p, BackRec q,
         return;
     }
     // Longer rows: the same arithmetic in three batched passes (base; update,
-    // with cur holding the unnormalised value; normalisation).
+    // with cur holding the unnormalised value; normalisation). A config without
+    // actions comes here too: it owns no cell, and no pass reads or writes one.
     float base = 0.0f;
     for (uint32_t c0 = 0; c0 < n; c0 += ROW_BATCH) {
         const uint32_t m = n - c0 < ROW_BATCH ? n - c0 : ROW_BATCH;
@@ -1291,7 +1292,7 @@ __global__ void k_normalize(WaveDev w, int touched0, int touched1) {
     AccRec q = decision_row(w, i, &p);
     uint32_t lo = q.lo, hi = q.lo + q.n;
     const bool touched = p ? touched1 : touched0;
-    if (q.n <= ROW_BATCH) {  // the row's loads issued together, then the same sum and quotients
+    if (q.n - 1 < ROW_BATCH) {  // 1 to 12 cells: the row's loads issued together, then the same sum and quotients
         const float* src = (touched ? scalar(w.sum) : scalar(w.cur)) + lo;
         const bool more[ROW_QUADS] = {true, q.n > 4, q.n > 8};
         float x[ROW_QUADS][4];
@@ -1304,10 +1305,10 @@ __global__ void k_normalize(WaveDev w, int touched0, int touched1) {
             if (more[h])
 #pragma unroll
                 for (uint32_t k = 0; k < 4; k++) s = 4 * h + k < q.n ? s + x[h][k] : s;
-        const float u = 1.0f / (float)(q.n ? q.n : 1);
+        const float u = 1.0f / (float)q.n;
 #pragma unroll
         for (uint32_t h = 0; h < ROW_QUADS; h++)
-            if (more[h] && q.n) {
+            if (more[h]) {
 #pragma unroll
                 for (uint32_t k = 0; k < 4; k++) {
                     const float y = s > 0.0f ? x[h][k] / s : u;
