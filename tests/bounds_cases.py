@@ -81,3 +81,26 @@ def cases(wave):
     else:
         raise AssertionError("no unit has reach rows at its deepest level, value rows and leaves")
     return out
+
+
+def split_parents(wave):
+    """Edits, as above, that leave a unit's reach row with parent slots on both sides of its reach window, every one
+    inside written before it is read: the row's base moved to the window's last slot with all it reads past it, or
+    from the window's first slot to the one before."""
+    a = wave.array
+    reach_len = wave.stats()["reach_len"]
+    units, out = a("units").reshape(-1, UNIT_WORDS), {}
+    for p in (0, 1):
+        rec, lvl = a(f"reach_rec{p}").reshape(-1, REC_WORDS), a(f"reach_lvl{p}")
+        for u in units:
+            rwin, rn, l0, nl = int(u[U_RWIN0 + p]), int(u[U_RWIN_N0 + p]), int(u[U_LVL0]), int(u[U_NLEVELS])
+            for x in range(int(lvl[l0]), int(lvl[l0 + nl])):
+                _, pbase, start, kn = rec[x].tolist()
+                src = a("rvd_src" if kn >> 31 else "rev_src")[start:start + (kn & 0x1FFFFFFF)]
+                word = (f"reach_rec{p}", REC_WORDS * x + 1)
+                if len(src) and src.min() > 0 and src.max() < reach_len - (rwin + rn - 1):
+                    out.setdefault((p, "past"), (*word, rwin + rn - 1, "unit reach row partly inside its reach window"))
+                if len(src) and src.max() > 0 and pbase == rwin > 0:
+                    out.setdefault((p, "before"), (*word, rwin - 1, "unit reach row partly inside its reach window"))
+    assert len(out) == 4
+    return list(out.values())

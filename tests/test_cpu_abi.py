@@ -246,6 +246,22 @@ def test_host_check_names_the_first_failing_condition(monkeypatch):
         plain.array("no_such_table")
 
 
+def test_host_check_refuses_a_reach_row_with_parents_on_both_sides_of_the_window(monkeypatch):
+    """The unit kernels ask of a reach row's first parent slot only whether it lies in the unit's LDS window and
+    read the others from the same side."""
+    import bounds_cases as B
+
+    monkeypatch.setenv("WC_UNIT_SLOTS", B.UNIT_SLOTS)
+    wave = ww.Wave(B.jobs())
+    for name, index, value, msg in B.split_parents(wave):
+        old = int(wave.array(name)[index])
+        wave.poke(name, index, value)
+        with pytest.raises(ww.WaveError, match="^wave bounds: " + re.escape(msg) + "$"):
+            wave.check()
+        wave.poke(name, index, old)
+        wave.check()
+
+
 def test_host_check_survives_random_single_word_edits(monkeypatch):
     """Random single-word edits of every table wc_wave_array names: the host
     check accepts the wave or refuses it with "wave bounds: ...", and never

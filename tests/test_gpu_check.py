@@ -68,6 +68,21 @@ def test_device_check_names_what_the_host_names(monkeypatch):
         wave.check(ex, v)
 
 
+def test_device_check_refuses_parents_on_both_sides_of_the_window(monkeypatch):
+    monkeypatch.setenv("WC_UNIT_SLOTS", B.UNIT_SLOTS)
+    wave = ww.Wave(B.jobs())
+    ex, v = executor_for("wave256")
+    for name, index, value, msg in B.split_parents(wave):
+        say(f"[check] {name}[{index}] = {value}: expect {msg!r}")
+        old = int(wave.array(name)[index])
+        wave.poke(name, index, value)
+        with pytest.raises(ww.WaveError) as dev:
+            wave.check(ex, v)
+        assert str(dev.value) == "wave bounds: " + msg
+        wave.poke(name, index, old)
+        wave.check(ex, v)
+
+
 def test_an_edited_wave_is_refused_before_its_schedule(monkeypatch):
     monkeypatch.setenv("WC_UNIT_SLOTS", B.UNIT_SLOTS)
     jobs = B.jobs()[:2]

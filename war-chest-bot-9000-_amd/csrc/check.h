@@ -12,8 +12,9 @@
 // cells' value slots, the network rows and their config lists, the pool
 // groups (bounds, shared lists, every row in exactly one group), every row
 // record and the elements it names, the two-tower blocks' rows, and each
-// subtree unit's windows (its rows write and read inside them; a reach row
-// reads a window slot only after a shallower level wrote it). The lists only
+// subtree unit's windows (its rows write and read inside them; a reach row's
+// parent slots are all inside or all outside, and it reads one inside only
+// after a shallower level wrote it). The lists only
 // the host reads (node CSR, task lists) are not uploaded and not checked here.
 #pragma once
 
@@ -50,6 +51,7 @@ enum CheckCode : uint32_t {
     CK_LEAF_REC,
     CK_TOWER_CONFIGS,
     CK_UNIT_RWIN,
+    CK_UNIT_SPLIT,
     CK_UNIT_UNWRITTEN,
     CK_UNIT_WRITES_OUT,
     CK_UNIT_LEAF_OUT,

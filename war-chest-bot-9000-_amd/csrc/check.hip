@@ -209,8 +209,9 @@ __global__ __launch_bounds__(CBLOCK) void k_check_tower(CheckArgs a, int p) {
 }
 
 // One workgroup per subtree unit. The kernels keep a unit's windows in LDS:
-// each of its reach rows, level by level, may read a window slot only after
-// a shallower level wrote it (a bitmap of the window's slots in LDS, a
+// each of its reach rows has all its parent slots inside the window or all
+// outside (the kernel asks of the parent's first slot only) and, level by
+// level, may read a window slot only after a shallower level wrote it (a bitmap of the window's slots in LDS, a
 // barrier between the reads and the writes of a level) and writes inside the
 // window; its leaves, terminals and value rows write and read inside its
 // value window. The unit's own level and leaf ranges were checked on the host.
@@ -234,14 +235,16 @@ __global__ __launch_bounds__(CBLOCK) void k_check_units(CheckArgs a) {
                     const uint64_t n = r.kn & REC_N;
                     const bool rev = (r.kn >> 31) == REACH_REV;
                     if (r.start + n > (rev ? a.rev_n : a.rvd_n)) continue;  // the record check reports it
+                    const bool inside = (uint64_t)r.pbase - rlo < rn;
+                    bool split = false, early = false;
                     for (uint64_t k = 0; k < n; k++) {
                         const uint64_t i = (uint64_t)r.pbase + (rev ? a.w.rev_src[r.start + k] : a.w.rvd_src[r.start + k]);
                         const uint64_t s = i - rlo;
-                        if (s < rn && !((written[s >> 5] >> (s & 31)) & 1u)) {
-                            raise_flag(a, CK_UNIT_UNWRITTEN);
-                            break;
-                        }
+                        split |= (s < rn) != inside;
+                        if (s < rn) early |= !((written[s >> 5] >> (s & 31)) & 1u);
                     }
+                    if (split) raise_flag(a, CK_UNIT_SPLIT);
+                    if (early) raise_flag(a, CK_UNIT_UNWRITTEN);
                 }
                 __syncthreads();
                 for (uint32_t x = b + t; x < e; x += nt) {
@@ -319,6 +322,7 @@ const char* check_message(uint32_t code) {
         "leaf record",
         "tower block configs",
         "unit reach window",
+        "unit reach row partly inside its reach window",
         "unit reach row reads an unwritten window slot",
         "unit reach row writes outside its reach window",
         "unit leaf outside its value window",

@@ -1960,8 +1960,10 @@ bool validate_elements(const WaveHost& w, std::string* err) {
     auto unit_check = [&](uint64_t ui) -> const char* {
         const UnitDev& u = w.units[ui];
         for (int p = 0; p < 2; p++) {
-            // The reach window: the unit's rows write inside it, and a row reads
-            // a slot inside it only once a shallower level has written it.
+            // The reach window: the unit's rows write inside it, a row's parent
+            // slots are all inside it or all outside (the kernel takes the
+            // parent's first slot for all of them), and a row reads a slot
+            // inside it only once a shallower level has written it.
             const uint64_t rlo = u.rwin[p], rn = u.rwin_n[p];
             if (rlo + rn > w.reach_len) return "unit reach window";
             std::vector<uint8_t> written(rn, 0);
@@ -1970,11 +1972,15 @@ bool validate_elements(const WaveHost& w, std::string* err) {
                 for (uint32_t x = b; x < e; x++) {
                     const ReachRec& r = w.reach_rec[p][x];
                     const uint32_t n = r.kn & REC_N;
+                    const bool inside = uint64_t(r.pbase) - rlo < rn;
+                    bool early = false;
                     for (uint32_t k = 0; k < n; k++) {
                         const uint64_t i = uint64_t(r.pbase) +
                                            ((r.kn >> 31) == REACH_REV ? w.rev_src[r.start + k] : w.rvd_src[r.start + k]);
-                        if (i - rlo < rn && !written[i - rlo]) return "unit reach row reads an unwritten window slot";
+                        if ((i - rlo < rn) != inside) return "unit reach row partly inside its reach window";
+                        early |= inside && !written[i - rlo];
                     }
+                    if (early) return "unit reach row reads an unwritten window slot";
                 }
                 for (uint32_t x = b; x < e; x++) {
                     const uint64_t o = w.reach_rec[p][x].out;
