@@ -328,13 +328,14 @@ int wc_mlp_forward(wc_executor* ex, uint64_t version, uint32_t rows, const float
 /* No counterpart in the reference: for callers that cannot allocate device
  * memory (code under HIP graph capture, tight serving loops, harnesses that
  * forbid hipMalloc). wc_mlp_forward on device-resident buffers -- x: rows x in
- * f32, out: rows x heads f32 -- with every intermediate it needs (a
- * layer-by-layer net's input operand and hidden activations) in one fixed
- * device array of WC_NOALLOC_SCRATCH_BYTES per GPU, held until the process
- * ends; the call makes no device allocation. stream NULL: queued on the executor's stream
+ * f32, out: rows x heads f32; they may overlap -- with every intermediate it
+ * needs (a layer-by-layer net's hidden activations, the input operand there and
+ * for buffers that overlap) in one fixed device array of
+ * WC_NOALLOC_SCRATCH_BYTES per GPU, held until the process ends; the call makes
+ * no device allocation. stream NULL: queued on the executor's stream
  * and the call waits for the result; otherwise queued on that hipStream_t and
- * the call returns at once. Calls that overlap on one GPU share the array and
- * race. Fails (WC_ERR_INVALID) when the rows need more than the array holds
+ * the call returns at once. Calls that overlap in time on one GPU share the
+ * array and race. Fails (WC_ERR_INVALID) when the rows need more than the array holds
  * (about 32k rows of a 512-input 16-bit net, 8k of the float32 net). */
 #define WC_NOALLOC_SCRATCH_BYTES (32u << 20)
 int wc_mlp_forward_noalloc(wc_executor* ex, uint64_t version, uint32_t rows, const float* x, float* out,

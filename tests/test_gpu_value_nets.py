@@ -88,6 +88,32 @@ def test_fused_net_from_rows_equals_the_planned_passes(precision, inputs, hidden
     np.testing.assert_array_equal(got, want)
 
 
+# in place, out ahead of and behind x by part of a row and by many rows, and end to end; shared head columns,
+# one pass and many, rows more and less wide than the head
+@pytest.mark.parametrize("precision", [ww.WC_F16, ww.WC_BF16, ww.WC_F16X, ww.WC_PRECISE])
+@pytest.mark.parametrize("inputs,hidden,layers,heads,rows,xo,oo", [
+    (512, 384, 3, 567, 250, 0, 0), (512, 384, 3, 64, 5000, 0, 0), (96, 128, 2, 567, 3000, 40, 0),
+    (480, 384, 3, 22, 4000, 0, 100), (512, 384, 3, 64, 5000, 160000, 0), (160, 64, 1, 33, 700, 0, 160 * 700)])
+def test_net_on_overlapping_buffers(precision, inputs, hidden, layers, heads, rows, xo, oo):
+    say(f"case overlap {precision}: {rows} rows, {inputs} -> {layers}x{hidden} -> {heads}, x + {xo}, out + {oo} floats")
+    net = ww.synth_weights(ww.mlp_dims(inputs, hidden, layers, heads, pool=8), seed=rows)
+    x = ww.synth_features(rows, inputs, seed=rows + 1)
+    ex = ww.Executor(0, precision)
+    v = ex.publish(net)
+    hip = Hip()
+    at = hip.alloc(4 * max(xo + rows * inputs, oo + rows * heads))
+    got = np.zeros((rows, heads), np.float32)
+    try:
+        hip.to_dev(at + 4 * xo, x)
+        ex.mlp_noalloc(v, rows, at + 4 * xo, at + 4 * oo)
+        hip.to_host(got, at + 4 * oo)
+        want = ex.mlp(v, x, heads=heads)
+    finally:
+        hip.free(at)
+        ex.close()
+    np.testing.assert_array_equal(got, want)
+
+
 # one to four row blocks per pass, two rounds of passes, widths that leave wavefronts idle
 @pytest.mark.parametrize("inputs,hidden,layers,heads,rows,offset", [
     (512, 384, 3, 567, 1, 0), (32, 32, 1, 1, 17, 1), (160, 352, 8, 130, 250, 3), (512, 384, 3, 22, 5100, 0),

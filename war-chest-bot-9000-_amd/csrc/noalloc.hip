@@ -30,6 +30,27 @@ void* g_scratch[MAX_DEVICES] = {};  // the array's device address on each device
 
 size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
 
+// Passes of up to CHAIN_PASS_BLOCKS consecutive 16-row blocks, every pass
+// computing all `cols` head columns, written on the device (no host buffer, no
+// copy).
+__global__ void k_plan_consecutive(ChainPass* plan, uint32_t nrb, uint32_t cols) {
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t npass = (nrb + CHAIN_PASS_BLOCKS - 1) / CHAIN_PASS_BLOCKS;
+    if (i >= npass) return;
+    ChainPass ps;
+    ps.n = min(CHAIN_PASS_BLOCKS, nrb - i * CHAIN_PASS_BLOCKS);
+    for (uint32_t j = 0; j < CHAIN_PASS_BLOCKS; j++) ps.rb[j] = j < ps.n ? i * CHAIN_PASS_BLOCKS + j : 0u;
+    ps.cols = cols;
+    ps.pad[0] = ps.pad[1] = 0;
+    plan[i] = ps;
+}
+
+// Whether `n` floats at a and `m` floats at b share memory.
+bool overlap(const float* a, size_t n, const float* b, size_t m) {
+    const uintptr_t x = (uintptr_t)a, y = (uintptr_t)b;
+    return x < y + 4 * m && y < x + 4 * n;
+}
+
 }  // namespace
 
 // The scratch array's address on `device`, looked up the first time a device
@@ -67,12 +88,17 @@ bool Executor::mlp_forward_noalloc(uint64_t version, uint32_t rows, const float*
         return false;
     }
     if (rows == 0) return true;
-    // The pieces of one call, 256-byte aligned: the 16-bit input operand (rows
-    // padded to GEMM_ROWS; compensated f16: hi and lo planes) and the hidden
-    // activations of the layer-by-layer nets. The fused net needs no scratch,
-    // but keeps the bound its callers size their batches by: its operand and
-    // 48 bytes per 128 rows, or (compensated f16) the layer-by-layer pieces.
-    const bool fused = precision_ != WC_PRECISE && chain_fits(ns.in, ns.hidden, ns.layers);
+    // The fused net reads x while its workgroups write out, so it takes buffers
+    // that share no memory, and no scratch. Where they do, x is first copied
+    // into scratch as the 16-bit operand: then the passes of a plan read that
+    // (f16, bf16), or the layers run one by one (compensated f16).
+    const bool chain = precision_ != WC_PRECISE && chain_fits(ns.in, ns.hidden, ns.layers);
+    const bool fused = chain && !overlap(x, size_t(rows) * ns.in, out, size_t(rows) * ns.heads);
+    const bool planned = chain && precision_ != WC_F16X;
+    // The pieces of one call, 256-byte aligned: the pass plan, the 16-bit input
+    // operand (rows padded to GEMM_ROWS; compensated f16: hi and lo planes), the
+    // hidden activations of the layer-by-layer nets. One bound for every call of
+    // a network, which callers size their batches by, whether it needs them or not.
     const size_t esz = precision_ == WC_F16X ? 4 : 2;
     const size_t prow = precision_ == WC_PRECISE ? rows : gemm_rows(rows);
     const uint32_t nrb = (rows + 15) / 16, npass = (nrb + CHAIN_PASS_BLOCKS - 1) / CHAIN_PASS_BLOCKS;
@@ -82,11 +108,10 @@ bool Executor::mlp_forward_noalloc(uint64_t version, uint32_t rows, const float*
         at = a + bytes;
         return a;
     };
-    if (fused && precision_ != WC_F16X) take(size_t(npass) * sizeof(ChainPass));
+    const size_t o_plan = planned ? take(size_t(npass) * sizeof(ChainPass)) : 0;
     const size_t o_x = precision_ == WC_PRECISE ? 0 : take(prow * ns.in * esz);
     const size_t hbytes = prow * ns.hidden * (precision_ == WC_PRECISE ? 4 : esz);
-    const bool acts = !fused || precision_ == WC_F16X;
-    const size_t o_h0 = acts ? take(hbytes) : 0, o_h1 = acts ? take(hbytes) : 0;
+    const size_t o_h0 = planned ? 0 : take(hbytes), o_h1 = planned ? 0 : take(hbytes);
     if (at > WC_NOALLOC_SCRATCH_BYTES) {
         const size_t per_row = std::max<size_t>(at / std::max<uint32_t>(rows, 1), 1);
         *err = std::to_string(rows) + " rows need " + std::to_string(at) + " bytes of scratch; the allocation-free "
@@ -116,15 +141,21 @@ bool Executor::mlp_forward_noalloc(uint64_t version, uint32_t rows, const float*
     } else {
         void* xop = base + o_x;
         launch_to16(precision_, x, xop, rows, ns.in, false, s);
-        const void* in = xop;
-        uint32_t k = ns.in;
-        for (uint32_t l = 0; l < ns.layers; l++) {
-            void* o = base + (l & 1 ? o_h1 : o_h0);
-            launch_gemm16(precision_, in, k, bank->W[l], bank->B[l], ns.hidden, o, rows, true, true, s);
-            in = o;
-            k = ns.hidden;
+        if (planned) {
+            ChainPass* plan = (ChainPass*)(base + o_plan);
+            hipLaunchKernelGGL(k_plan_consecutive, dim3((npass + 63) / 64), dim3(64), 0, s, plan, nrb, ns.heads);
+            launch_chain(precision_, chain_net(*bank), xop, rows, out, plan, npass, s);
+        } else {
+            const void* in = xop;
+            uint32_t k = ns.in;
+            for (uint32_t l = 0; l < ns.layers; l++) {
+                void* o = base + (l & 1 ? o_h1 : o_h0);
+                launch_gemm16(precision_, in, k, bank->W[l], bank->B[l], ns.hidden, o, rows, true, true, s);
+                in = o;
+                k = ns.hidden;
+            }
+            launch_gemm16(precision_, in, ns.hidden, bank->Whead, bank->bhead, ns.heads, out, rows, false, false, s);
         }
-        launch_gemm16(precision_, in, ns.hidden, bank->Whead, bank->bhead, ns.heads, out, rows, false, false, s);
     }
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) {
