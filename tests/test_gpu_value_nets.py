@@ -5,6 +5,7 @@ dispatch takes (few, some and many rows), with inputs, hidden widths and heads
 that fill no tile, no 16-byte run and no k tile, from buffers that 16-byte
 loads may not read, and with infinite weights behind zero inputs.
 """
+import ctypes as C
 import sys
 
 import numpy as np
@@ -69,6 +70,25 @@ def test_float32_net_skips_zero_inputs_of_infinite_weights():
     want = O.mlp(x, keys, net, O.NET_F32)
     assert np.isfinite(want[:25]).all() and not np.isfinite(want[25:]).all()
     np.testing.assert_array_equal(got, want)
+
+
+def test_float32_bank_holds_its_weights_once():
+    """Device memory a published float32 network takes: its matrices and biases, and no copy of them beside."""
+    say("case float32 bank: device memory of a 2048 -> 3x2048 -> 64 net")
+    net = ww.synth_weights(ww.mlp_dims(2048, 2048, 3, 64, pool=8), seed=1)
+    size = 4 * (net.w.size + net.b.size)
+    ex = ww.Executor(0, ww.WC_PRECISE)
+    ex.publish(ww.synth_weights(ww.mlp_dims(32, 32, 1, 1, pool=8), seed=1))  # (what a first publish sets up)
+    free, total = C.c_size_t(), C.c_size_t()
+    L = Hip().L
+    L.hipMemGetInfo.argtypes, L.hipMemGetInfo.restype = [C.POINTER(C.c_size_t)] * 2, C.c_int
+    assert L.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    before = free.value
+    ex.publish(net)
+    assert L.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    ex.close()
+    say(f"  {size} bytes of weights, {before - free.value} bytes of memory")
+    assert size <= before - free.value < 1.25 * size
 
 
 # one pass per row block, several blocks per pass with a short last one, full passes; buffers off 16 bytes

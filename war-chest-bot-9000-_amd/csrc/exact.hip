@@ -201,21 +201,6 @@ void dispatch(bool head, bool skip, const float* X, uint32_t K, const float* Wt,
 
 }  // namespace
 
-// dst[n, k] = src[k, n] (src [K x N]) when transposed, else a copy.
-__global__ void k_rows(const float* __restrict__ src, float* __restrict__ dst, uint32_t N, uint32_t K,
-                       int transposed) {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (size_t)N * K) return;
-    dst[i] = src[transposed ? i % K * N + i / K : i];
-}
-
-void launch_rows(const float* src, float* dst, uint32_t N, uint32_t K, bool transposed, hipStream_t s) {
-    const size_t n = (size_t)N * K;
-    if (n)
-        hipLaunchKernelGGL(k_rows, dim3((uint32_t)((n + THREADS - 1) / THREADS)), dim3(THREADS), 0, s, src, dst, N, K,
-                           (int)transposed);
-}
-
 void launch_dense_exact(const float* X, uint32_t K, const float* Wt, const float* b, uint32_t N, float* Y,
                         uint32_t rows, bool skip, hipStream_t s) {
     dispatch(false, skip, X, K, Wt, b, N, Y, rows, nullptr, s);

@@ -272,6 +272,25 @@ uint64_t Executor::publish_v5(const NetShape& ns, const float* w, size_t nw, con
     return bank.version;
 }
 
+// dst[n, k] = src[k, n] (src [K x N]) when transposed, else a copy.
+static void rows_of(const float* src, float* dst, size_t N, size_t K, bool transposed) {
+    if (!transposed) {
+        std::memcpy(dst, src, N * K * 4);
+        return;
+    }
+    constexpr size_t STRIP = 64, TILE = 16;  // rows per task, and a cache line of each side
+    parallel_for(
+        (N + STRIP - 1) / STRIP,
+        [&](size_t strip) {
+            const size_t end = std::min(N, (strip + 1) * STRIP);
+            for (size_t k0 = 0; k0 < K; k0 += TILE)
+                for (size_t n0 = strip * STRIP; n0 < end; n0 += TILE)
+                    for (size_t n = n0; n < std::min(n0 + TILE, end); n++)
+                        for (size_t k = k0; k < std::min(k0 + TILE, K); k++) dst[n * K + k] = src[k * N + n];
+        },
+        8);
+}
+
 uint64_t Executor::publish(const NetShape& ns, const std::vector<uint32_t>& dims, const float* w, size_t nw,
                            const float* b, size_t nb, std::string* err, const float* ln, size_t nln) {
     if (ns.kind == MODEL_V5) return publish_v5(ns, w, nw, b, nb, ln, nln, err);
@@ -349,8 +368,18 @@ uint64_t Executor::publish(const NetShape& ns, const std::vector<uint32_t>& dims
     at = align256(at + nb * 4);
     const size_t roff = at;  // readout weight (two-tower), f32
     if (tower) at = align256(at + size_t(ns.hidden) * 4);
-    // Staging for the conversion to the stored layout on the device.
-    const size_t stage = at, total = at + nw * 4;
+    // Staging for f32 -> 16-bit conversion on the device (float32 banks are laid
+    // out here: their staging would double what they hold).
+    const size_t stage = at, total = at + (precision_ == WC_PRECISE ? 0 : nw * 4);
+    std::unique_ptr<float[]> laid;
+    if (precision_ == WC_PRECISE) {
+        laid.reset(new float[mats_end / 4]);  // (first touched by the threads that fill it)
+        size_t from = 0;
+        for (size_t k = 0; k < mats.size(); k++) {
+            rows_of(w + from, laid.get() + moff[k] / 4, mats[k].n, mats[k].k, !mats[k].head);
+            from += mats[k].k * mats[k].n;
+        }
+    }
     void* mem = nullptr;
     if (hipMalloc(&mem, total) != hipSuccess) {
         *err = "hipMalloc of the weight bank failed";
@@ -359,8 +388,8 @@ uint64_t Executor::publish(const NetShape& ns, const std::vector<uint32_t>& dims
     char* base = (char*)mem;
     bool okc = hipMemcpyAsync(base + boff, b, nb * 4, hipMemcpyHostToDevice, stream_) == hipSuccess;
     size_t src = 0;
-    okc = okc && hipMemcpyAsync(base + stage, w, nw * 4, hipMemcpyHostToDevice, stream_) == hipSuccess;
     if (precision_ == WC_PRECISE) {
+        okc = okc && hipMemcpyAsync(base, laid.get(), mats_end, hipMemcpyHostToDevice, stream_) == hipSuccess;
         // (as integers: the comparison vectorises)
         const uint32_t inf = 0x7f800000u;
         uint32_t bad = 0;
@@ -370,12 +399,9 @@ uint64_t Executor::publish(const NetShape& ns, const std::vector<uint32_t>& dims
             bad |= (u & inf) == inf ? 1u : 0u;
         }
         bank.skip = bad != 0;
-        for (size_t k = 0; k < mats.size(); k++) {
-            launch_rows((const float*)(base + stage) + src, (float*)(base + moff[k]), (uint32_t)mats[k].n,
-                        (uint32_t)mats[k].k, !mats[k].head, stream_);
-            src += mats[k].k * mats[k].n;
-        }
+        for (const Mat& m : mats) src += m.k * m.n;
     } else {
+        okc = okc && hipMemcpyAsync(base + stage, w, nw * 4, hipMemcpyHostToDevice, stream_) == hipSuccess;
         okc = okc && hipMemsetAsync(base, 0, mats_end, stream_) == hipSuccess;  // row padding
         for (size_t k = 0; k < mats.size(); k++) {
             const size_t n = mats[k].k * mats[k].n;

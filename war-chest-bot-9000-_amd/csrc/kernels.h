@@ -140,9 +140,6 @@ void launch_collect_root(const WaveDev& w, int root, int player, hipStream_t s);
 // Leaf MLP.
 // Exact float32 layers (exact.hip), in the CPU loop order; Wt holds one
 // K-contiguous row per output.
-// launch_rows lays a weight matrix out so: from [K x N] when transposed, else
-// from [N x K].
-void launch_rows(const float* src, float* dst, uint32_t N, uint32_t K, bool transposed, hipStream_t s);
 // Y = relu(X Wt^T + b). skip: leave out zero inputs' terms, as the CPU loop
 // does (needed for a bank with an infinite or NaN weight, NetBank::skip).
 void launch_dense_exact(const float* X, uint32_t K, const float* Wt, const float* b, uint32_t N, float* Y,
