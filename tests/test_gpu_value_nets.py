@@ -108,6 +108,25 @@ def test_fused_net_from_rows_equals_the_planned_passes(precision, inputs, hidden
     np.testing.assert_array_equal(got, want)
 
 
+# the same launches against the oracle's model of the operand rounding (which shares nothing with them), within the
+# bounds of the other comparisons with it: the products' float32 sums run in another order, and where that moves an
+# activation across a rounding boundary it moves by one unit of the operand's last place
+@pytest.mark.parametrize("precision,mode,bound", [(ww.WC_F16, O.NET_F16, 2e-3), (ww.WC_BF16, O.NET_BF16, 1e-2)])
+@pytest.mark.parametrize("inputs,hidden,layers,heads,rows,offset", [
+    (512, 384, 3, 567, 250, 3), (96, 352, 2, 130, 1713, 0), (480, 128, 8, 64, 2100, 2), (512, 384, 3, 22, 33, 1)])
+def test_fused_net_from_rows_tracks_the_operand_model(precision, mode, bound, inputs, hidden, layers, heads, rows,
+                                                      offset):
+    say(f"case fused net {precision} against the model: {rows} rows, {inputs} -> {layers}x{hidden} -> {heads}")
+    net = ww.synth_weights(ww.mlp_dims(inputs, hidden, layers, heads, pool=8), seed=rows)
+    x = ww.synth_features(rows, inputs, seed=rows + 1)
+    ex = ww.Executor(0, precision)
+    got = forward_on_device(ex, ex.publish(net), x, heads, offset)
+    ex.close()
+    want = O.mlp(x, np.tile(np.arange(heads, dtype=np.uint32), (rows, 1)), net, mode)
+    say(f"  max error {np.abs(got - want).max() / np.abs(want).max():.1e} of the largest value")
+    assert np.abs(got - want).max() <= bound * np.abs(want).max()
+
+
 # in place, out ahead of and behind x by part of a row and by many rows, and end to end; shared head columns,
 # one pass and many, rows more and less wide than the head
 @pytest.mark.parametrize("precision", [ww.WC_F16, ww.WC_BF16, ww.WC_F16X, ww.WC_PRECISE])
