@@ -47,3 +47,26 @@ def test_pool_list_edges(precision, mode, bound, info, pool):
             np.testing.assert_allclose(mass.reshape(-1), ref_mass.reshape(-1), rtol=2e-6, atol=1e-30)
     wave.close()
     ex.close()
+
+
+@pytest.mark.parametrize("info,pool", [(1, 20), (17, 72), (64, 64), (81, 12), (257, 130)])
+def test_float32_pool_with_wide_offsets(monkeypatch, info, pool):
+    """The path of an embedding table of 4 GiB or more (WC_EMB_WIDE=1 forces it), against the oracle's leaf probe."""
+    print(f"case wide pool: lists of up to {info} configs, {pool} pooled columns", flush=True)
+    sys.stdout.flush()
+    monkeypatch.setenv("WC_EMB_WIDE", "1")
+    dims = ww.mlp_dims(inputs=300, hidden=64, layers=1, heads=max(info, 2), pool=pool)
+    jobs = ww.synth_jobs(dims, seed=info, trees=3, nodes_lo=20, nodes_hi=40, act_lo=2, act_hi=5, collapse=0.6,
+                         chance=1, draw_lo=2, draw_hi=3, info_fixed=info, dirichlet=1, iters=2, depth=2, snapshots=1,
+                         nroots=1, **W.DCFR)
+    net = ww.synth_weights(dims, seed=info + 1)
+    ex = ww.Executor(0, ww.WC_PRECISE)
+    v = ex.publish(net)
+    wave = ww.Wave(jobs)
+    for p in (0, 1):
+        got, mass = ex.leaf_probe(wave, v, p)
+        want = [O.leaf_probe(j, net, O.NET_F32, p) for j in jobs]
+        np.testing.assert_array_equal(got, np.concatenate([a for a, _ in want]))
+        np.testing.assert_array_equal(mass.reshape(-1), np.concatenate([m for _, m in want]).reshape(-1))
+    wave.close()
+    ex.close()

@@ -123,6 +123,7 @@ Executor::Executor(int device, int precision) : device_(device), precision_(prec
     if (const char* env = std::getenv("WC_CHAIN_SPLIT")) split_ = std::strcmp(env, "0") != 0;
     if (const char* env = std::getenv("WC_GRAPH")) graph_ = std::strcmp(env, "1") == 0;
     if (const char* env = std::getenv("WC_UNIT_LDS")) unit_lds_ = std::strcmp(env, "0") != 0;
+    if (const char* env = std::getenv("WC_EMB_WIDE")) emb_wide_ = std::strcmp(env, "1") == 0;
     if (const char* env = std::getenv("WC_V5_SCALAR")) v5_scalar_ = std::strcmp(env, "1") == 0;
     ok_ = true;
 }
@@ -668,7 +669,7 @@ bool Executor::upload(const WaveHost& w, const NetBank& bank, uint32_t slot, std
     d.max_rwin = w.max_rwin;
     d.unit_lds = unit_lds_ ? 1u : 0u;
     d.nsub = w.nsub;
-    d.emb_wide = uint64_t(ncfg) * ns.pool * 4 > UINT32_MAX ? 1u : 0u;
+    d.emb_wide = emb_wide_ || uint64_t(ncfg) * ns.pool * 4 > UINT32_MAX ? 1u : 0u;
     d.regret = (float*)(A + a_regret);
     d.cur = (float*)(A + a_cur);
     d.sum = (float*)(A + a_sum);

@@ -303,6 +303,9 @@ class Executor {
     // WC_UNIT_LDS=0: the sweep and reach passes read and write unit windows in
     // HBM only (the paths taken when a window does not fit LDS)
     bool unit_lds_ = true;
+    // WC_EMB_WIDE=1: the float32 pooling takes 64-bit embedding offsets (the
+    // path taken when the table reaches 4 GiB)
+    bool emb_wide_ = false;
     // WC_V5_SCALAR=1: the v5 network's 16-bit path without the matrix cores
     // (rounded operands, float32 sums in ascending order)
     bool v5_scalar_ = false;
