@@ -2,8 +2,8 @@
 wc_mlp_forward, through the C ABI, on device-resident buffers.
 
 Two calls in a row, the second with fewer rows (the shared scratch keeps the
-first call's contents), in f16 (the fused net), float32 (the exact net) and
-compensated f16 (layer by layer): outputs bit-identical to wc_mlp_forward's.
+first call's contents), in f16 and compensated f16 (the fused nets) and float32
+(the exact net): outputs bit-identical to wc_mlp_forward's.
 Rows beyond the scratch are refused with an error naming it. The same two calls
 queued on a stream the caller created (the call returns at once; the caller
 synchronizes that stream) give the same outputs.
@@ -95,8 +95,7 @@ def test_noalloc_matches_mlp_forward_twice(precision):
 
 @pytest.mark.parametrize("precision", [ww.WC_F16, ww.WC_PRECISE])
 def test_noalloc_on_a_caller_stream(precision):
-    """Queued on the caller's own stream (the plan kernel and the net run there):
-    the call returns at once, and after the caller synchronizes that stream the
+    """Queued on the caller's own stream (the net runs there): the call returns at once, and after the caller synchronizes that stream the
     outputs equal wc_mlp_forward's, on two calls in a row, the second smaller."""
     hip = Hip()
     net = W.net_for("mlp65k")

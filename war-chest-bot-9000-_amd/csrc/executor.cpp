@@ -38,8 +38,9 @@ float cfr_factor(float t, float p) {
 size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
 
 // The table blob: arrays at 256-byte aligned offsets, laid out first, then
-// copied into pinned staging memory on several host threads (the upload is one
-// asynchronous copy from there). The sources must outlive copy_to.
+// copied into pinned staging memory on several host threads, a segment at a
+// time (the upload is an asynchronous copy of each from there). The sources
+// must outlive copy_to.
 struct Blob {
     struct Piece {
         const uint8_t* src;

@@ -107,6 +107,9 @@ struct ReachPair {
 };
 void launch_reach_pair(const WaveDev& w, const ReachPair& a, const ReachPair& b, const ReachPair& c, hipStream_t s);
 void launch_seed_sum(const WaveDev& w, hipStream_t s);
+// The leading groups of a player's list (longest config lists first) that the
+// 16-bit pooling gives a workgroup each.
+uint32_t pool_long_groups(const PoolGroup* grp, uint32_t n);
 // Leaf reach masses and pooled beliefs of one player (-1 = both), written into
 // the query inputs x0 (traverser 0) and x1 (traverser 1) in the operand precision.
 // With acc >= 0, the same launch also takes player acc's average-strategy
@@ -114,9 +117,6 @@ void launch_seed_sum(const WaveDev& w, hipStream_t s);
 // discount and this iteration's addition, search.rs:1770-1779,1818-1835), in
 // workgroups of their own: it reads only the final reach and cur, as the
 // leaf input does.
-// The leading groups of a player's list (longest config lists first) that the
-// 16-bit pooling gives a workgroup each.
-uint32_t pool_long_groups(const PoolGroup* grp, uint32_t n);
 void launch_pool(const WaveDev& w, int player, int precision, void* x0, void* x1, hipStream_t s, int acc = -1,
                  float ds = 1.0f);
 // Seat and public features of both query inputs (once per upload).

@@ -131,9 +131,9 @@ constexpr uint32_t LEAF_BATCH = 4;
 // One child config's reach: the reverse gather in stored order (the CPU's
 // scatter order, engine/src/serialize.rs:714-723). With LDSR the unit's reach
 // window [rw, rw + rn) is also kept in LDS at lr: parent reach inside it is
-// read from there (a parent's slots are all inside or all outside), and the
-// row's result goes to both.
-template <bool REV, bool INSIDE>
+// read from there (a parent's slots are all inside or all outside: the wave's
+// checks hold every row to it), and the row's result goes to both.
+template <bool REV>
 __device__ __forceinline__ float reach_sum(const WaveDev& w, const float* reach, const float* strat, uint32_t lo,
                                            uint32_t n, uint32_t base) {
     const uint32_t* esrc = (REV ? w.rev_src : w.rvd_src) + lo;
@@ -178,10 +178,9 @@ __device__ __forceinline__ void reach_row(const WaveDev& w, float* reach, const 
     float v;
     if (LDSR && q.pbase - rw < rn) {
         const uint32_t base = q.pbase - rw;
-        v = rev ? reach_sum<true, true>(w, lr, strat, lo, n, base) : reach_sum<false, true>(w, lr, strat, lo, n, base);
+        v = rev ? reach_sum<true>(w, lr, strat, lo, n, base) : reach_sum<false>(w, lr, strat, lo, n, base);
     } else {
-        v = rev ? reach_sum<true, false>(w, reach, strat, lo, n, q.pbase)
-                : reach_sum<false, false>(w, reach, strat, lo, n, q.pbase);
+        v = rev ? reach_sum<true>(w, reach, strat, lo, n, q.pbase) : reach_sum<false>(w, reach, strat, lo, n, q.pbase);
     }
     reach[q.out] = v;
     if (LDSR) lr[q.out - rw] = v;
@@ -782,7 +781,7 @@ __device__ __forceinline__ void pool_long(const WaveDev& w, const PoolGroup* grp
     constexpr int PER = (POOL_GROUP * POOL_CH + BLOCK - 1) / BLOCK;
     float rv[PER];
     uint32_t iv = 0xffffffffu;
-    const uint32_t cc = t % POOL_CH, r0 = t / POOL_CH;  // this thread's column, and its rows r0, r0 + 2, ...
+    const uint32_t cc = t % POOL_CH, r0 = t / POOL_CH;  // this thread's column, and its rows r0, r0 + 4, ...
     auto fetch = [&](uint32_t c0) {
         const uint32_t c = c0 + cc;
         if (t < POOL_CH) iv = c < n ? cfgs[c] : 0xffffffffu;

@@ -682,7 +682,7 @@ constexpr int JT_LD = JW + 8;        // LDS row stride of the 16-bit operand (ha
 constexpr int JT_RB = JT_ROWS / 16;  // row blocks per tile
 constexpr int JT_HLD = D + 8;        // LDS row stride of the output tile (halves)
 
-// Net::join for a 64-row tile on the matrix cores (16x16x32, 16-bit operands,
+// Net::join for a 32-row tile on the matrix cores (16x16x32, 16-bit operands,
 // f32 accumulate). Eight wavefronts: wavefront w owns one 16-column block of
 // the 128-wide residual stream z (in its accumulator registers) and two of
 // the 256-wide output. LayerNorm statistics are summed per row across the
@@ -699,8 +699,9 @@ template <int PREC>
 __global__ __launch_bounds__(JT_WAVES * 64) void k_join_mfma(Net net, uint32_t rows, const uint16_t* __restrict__ X,
                                                             const float* __restrict__ P, const float* __restrict__ Jp,
                                                             uint16_t* __restrict__ H) {
-    // The operand twice, so that the next norm may write one while a slower
-    // wavefront still reads the other; the output tile takes both at the end.
+    // The operand, at either half in turn (the barrier in row_stats already
+    // keeps a norm's writes behind the last product's reads); the output tile
+    // takes both halves at the end.
     __shared__ __attribute__((aligned(16))) uint16_t tA[2][JT_ROWS * JT_LD];
     __shared__ float part[JT_WAVES][JT_ROWS], part2[JT_WAVES][JT_ROWS];
     __shared__ __attribute__((aligned(16))) float stat[JT_WAVES][2][JT_ROWS];  // each wavefront's own copy
