@@ -116,3 +116,59 @@ def test_empty_rows_bit_exact(case, monkeypatch):
         np.testing.assert_array_equal(got.carries, want["carries"].astype(np.float16))
     wave.close()
     ex.close()
+
+
+def without_configs(job: bytes) -> bytes:
+    """The job's tree with no config at any node."""
+    d = wcj8.decode(job)
+    for name in ("cfg_off", "reach_off", "soff", "legal_off", "draw_off", "draw_row_start", "rev_start", "rvd_start",
+                 "leaf_coff", "snap_coff"):
+        d[name] = np.zeros_like(d[name])
+    for name in ("legal_action", "legal_child", "legal_trans", "cell_row", "draw_to", "draw_p", "rev_src", "rev_cell",
+                 "rvd_src", "rvd_p", "leaf_cidx", "cphi", "cplayer"):
+        d[name] = d[name][:0]
+    d["ncfg"] = d["ncells"] = 0
+    d["root"] = [r[:0] for r in d["root"]]
+    d["carried"] = [[r[:0] for r in c] for c in d["carried"]]
+    return wcj8.encode(d)
+
+
+def configless_jobs(pool):
+    """Jobs without configs, and their network: pooled columns past the end of such a wave's tables."""
+    dims = ww.mlp_dims(inputs=2 * pool + 8, hidden=16, layers=1, heads=3, pool=pool)
+    jobs = ww.synth_jobs(dims, seed=pool, trees=2, nodes_lo=20, nodes_hi=30, act_lo=2, act_hi=4, collapse=0.6, chance=1,
+                         draw_lo=1, draw_hi=3, info_fixed=3, dirichlet=1, iters=3, depth=2, snapshots=1, nroots=2,
+                         **W.DCFR)
+    return [without_configs(j) for j in jobs], jobs, ww.synth_weights(dims, seed=pool + 1)
+
+
+def test_jobs_without_configs_are_accepted():
+    for j in configless_jobs(64)[0]:
+        ww.job_validate(j)
+    wave = ww.Wave(configless_jobs(64)[0])  # (checks it)
+    assert wave.stats()["rows"] > 0 and wave.stats()["table_bytes"] < 1 << 16
+    wave.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("wide", ["0", "1"])
+def test_waves_without_configs_read_no_embedding(wide, monkeypatch):
+    """Their embedding table is empty, and so is every leaf's pooled belief; beside other jobs they change nothing."""
+    monkeypatch.setenv("WC_EMB_WIDE", wide)
+    bare, jobs, net = configless_jobs(20000)
+    print(f"case waves without configs, wide offsets {wide}", flush=True)
+    ex = ww.Executor(0, ww.WC_PRECISE)
+    v = ex.publish(net)
+    for wave_jobs in (bare, [bare[0], jobs[0], bare[1], jobs[1]]):
+        wave = ww.Wave(wave_jobs)
+        for p in (0, 1):
+            got, mass = ex.leaf_probe(wave, v, p)
+            want = [O.leaf_probe(j, net, O.NET_F32, p) for j in wave_jobs]
+            np.testing.assert_array_equal(got, np.concatenate([a for a, _ in want]))
+            np.testing.assert_array_equal(mass.reshape(-1), np.concatenate([m for _, m in want]).reshape(-1))
+        for got, job in zip(ex.solve(wave, v), wave_jobs):
+            want = O.solve(job, net, O.NET_F32)
+            np.testing.assert_array_equal(got.strategy, want["strategy"])
+            np.testing.assert_array_equal(got.root_values, want["roots"])
+        wave.close()
+    ex.close()

@@ -535,7 +535,8 @@ __global__ __launch_bounds__(BLOCK) void k_pool_exact(WaveDev w, int player, flo
         float acc = 0.0f;
         // 16 configs' embeddings per batch, one batch loading while the one
         // before it is added in config order. Lanes past the list hold config
-        // 0, so that a batch's loads need no branch.
+        // 0, so that a batch's loads need no branch (an empty list loads none:
+        // the wave may have no config at all).
         float e0[16], e1[16];
         const uint32_t kk = live ? k : 0u;
         auto index = [&](uint32_t c0) { return (c0 + lane < n ? cfgs[c0 + lane] : 0u) * (WIDE ? 1u : pool); };
@@ -562,7 +563,7 @@ __global__ __launch_bounds__(BLOCK) void k_pool_exact(WaveDev w, int player, flo
         };
         uint32_t cf = index(0);
         float beta = belief(0);
-        fetch(e0, cf, 0);
+        if (n) fetch(e0, cf, 0);
         for (uint32_t c0 = 0; c0 < n; c0 += 64) {
             const uint32_t left = n - c0, cn = index(c0 + 64);
             const float bn = belief(c0 + 64);
