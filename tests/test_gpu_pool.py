@@ -70,3 +70,35 @@ def test_float32_pool_with_wide_offsets(monkeypatch, info, pool):
         np.testing.assert_array_equal(mass.reshape(-1), np.concatenate([m for _, m in want]).reshape(-1))
     wave.close()
     ex.close()
+
+
+@pytest.mark.parametrize("precision,pool", [(ww.WC_F16, 64), (ww.WC_BF16, 20), (ww.WC_F16X, 72)])
+def test_long_lists_that_fill_the_device(precision, pool):
+    """More than 16 lists of over 192 configs per CU take a wavefront each instead of a workgroup: the same sums in the
+    same order, so a wave of them solves as its parts do, which have few enough for workgroups."""
+    print(f"case pool: long lists that fill the device, precision {precision}, {pool} pooled columns", flush=True)
+    sys.stdout.flush()
+    dims = ww.mlp_dims(inputs=160, hidden=32, layers=1, heads=567, pool=pool)
+    jobs = ww.synth_jobs(dims, seed=9, trees=110, nodes_lo=200, nodes_hi=250, act_lo=2, act_hi=3, collapse=0.2,
+                         chance=1, draw_lo=2, draw_hi=2, info_fixed=567, dirichlet=1, iters=2, depth=2, snapshots=1,
+                         nroots=1, **W.DCFR)
+    ex = ww.Executor(0, precision)
+    v = ex.publish(ww.synth_weights(dims, seed=pool))
+
+    def solve(part):
+        wave = ww.Wave(part)
+        lists = [wave.array(f"pool_grp{p}").reshape(-1, 36)[:, 1] for p in (0, 1)]
+        out = ex.solve(wave, v)
+        wave.close()
+        return out, [int((n > 192).sum()) for n in lists]
+
+    whole, long = solve(jobs)
+    assert min(long) > 16 * 256
+    for lo in range(0, len(jobs), 55):
+        part, long = solve(jobs[lo:lo + 55])
+        assert 1024 < max(long) < 16 * 256
+        for got, want in zip(whole[lo:], part):
+            np.testing.assert_array_equal(got.strategy, want.strategy)
+            np.testing.assert_array_equal(got.root_values, want.root_values)
+            np.testing.assert_array_equal(got.carries, want.carries)
+    ex.close()

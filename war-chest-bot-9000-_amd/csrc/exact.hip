@@ -28,7 +28,10 @@ constexpr uint32_t THREADS = 256, SIDE = 16;  // a SIDE x SIDE grid of threads o
 // 64 for a 384-wide layer, 564 of 64 x 32): 142 us with 64 x 32 tiles, 148 with
 // 32 x 32, 171 with 64 x 64; 8,000 rows (750 of 64 x 64): 206 us with 64 x 64
 // tiles, 231 with 32 x 32. The smallest tile's k tile: 60 rows take 28.6 us
-// with 128 inputs, 30.6 with 32, 33.5 with 256.
+// with 128 inputs, 30.6 with 32, 33.5 with 256. Lines at 256 / 512 / 1,024 tiles
+// over 100 to 8,000 rows (four runs within 2%): the same below 500 rows, then
+// 512 in front (567 heads, 1,700 rows 106 / 91 / 114 us, 3,001 170 / 142 / 146)
+// except near 5,600 rows (248 / 248 / 227).
 constexpr uint64_t MIN_TILES = 512;
 
 enum : uint32_t { VEC_X = 1, VEC_W = 2 };  // 16-byte loads of the operand are aligned

@@ -642,7 +642,7 @@ bool Executor::upload(const WaveHost& w, const NetBank& bank, uint32_t slot, std
         d.leaf_rec[p] = (const LeafRec*)(T + o.lr[p]);
         d.pool_grp[p] = (const PoolGroup*)(T + o.pg[p]);
         d.npool[p] = (uint32_t)w.pool_grp[p].size();
-        d.nlong[p] = pool_long_groups(w.pool_grp[p].data(), d.npool[p]);
+        d.nlong[p] = pool_long_groups(w.pool_grp[p].data(), d.npool[p], cus_);
         d.nleaf[p] = (uint32_t)w.leaf_rec[p].size();
         d.tower_blk[p] = (const TowerBlock*)(T + o.twb[p]);
         d.tower_unit[p] = (const TowerUnit*)(T + o.twu[p]);

@@ -108,8 +108,8 @@ struct ReachPair {
 void launch_reach_pair(const WaveDev& w, const ReachPair& a, const ReachPair& b, const ReachPair& c, hipStream_t s);
 void launch_seed_sum(const WaveDev& w, hipStream_t s);
 // The leading groups of a player's list (longest config lists first) that the
-// 16-bit pooling gives a workgroup each.
-uint32_t pool_long_groups(const PoolGroup* grp, uint32_t n);
+// 16-bit pooling gives a workgroup each on `cus` compute units.
+uint32_t pool_long_groups(const PoolGroup* grp, uint32_t n, uint32_t cus);
 // Leaf reach masses and pooled beliefs of one player (-1 = both), written into
 // the query inputs x0 (traverser 0) and x1 (traverser 1) in the operand precision.
 // With acc >= 0, the same launch also takes player acc's average-strategy

@@ -605,19 +605,28 @@ __global__ __launch_bounds__(BLOCK) void k_pool_exact(WaveDev w, int player, flo
 // A list of up to POOL_LONG configs takes one wavefront, all its loads of a
 // 64-config chunk in flight together. A longer one is a chain of chunks, each
 // with dependent loads (config indices, then embeddings), so it takes a whole
-// workgroup: the wavefronts split the dimensions (16 each, so that every sum
-// keeps its one order), share the reach and the indices through LDS, and the
-// next chunk's are on their way while the current one multiplies. Bound: the
-// latency of those loads with four wavefronts per SIMD (five spill). Leaf-input
-// time per wave, all lists on single wavefronts against long ones on
-// workgroups: 32 heavy-tailed subgames 12.0 -> 8.4 ms, 64 depth-1 subgames in
-// compensated f16 2.43 -> 1.35 ms, 256 depth-2 subgames 3.81 -> 3.61 ms.
+// workgroup, unless there are enough of them to fill the device: the wavefronts
+// split the dimensions (16 each, so that every sum keeps its one order), share
+// the reach and the indices through LDS, and the next chunk's are on their way
+// while the current one multiplies. Bound: the latency of those loads with four
+// wavefronts per SIMD (five spill). Leaf-input time per wave, all lists on
+// single wavefronts against long ones on workgroups: 32 heavy-tailed subgames
+// 11.8 -> 8.2 ms, 64 depth-1 subgames in compensated f16 2.43 -> 1.37 ms, 256
+// depth-2 subgames 3.50 -> 3.40 ms.
 
-// Configs past which a list takes a workgroup (256 depth-2 subgames: 3.74 ms
-// per wave from 128 on, 3.61 from 192, 3.75 from 256; below the line four
-// wavefronts wait for the loads of one or two chunks), and configs per LDS
-// chunk.
-constexpr uint32_t POOL_LONG = 192, POOL_CH = 64;
+// Configs past which a list takes a workgroup, and configs per LDS chunk. Below
+// the line four wavefronts wait for the loads of one or two chunks; from 128 to
+// 256 it hardly matters where it lies (whole schedules at 128 / 192 / 256, 12
+// runs each within 0.02 ms: 256 depth-2 subgames 18.48 / 18.32 / 18.23 ms, 64 of
+// them 8.31 / 8.33 / 8.40, 32 heavy-tailed ones 33.5 at each, 64 depth-1 ones in
+// compensated f16 6.94 / 6.93 / 6.94).
+// POOL_FILL: wavefronts a CU holds (four per SIMD). Lists that fill the device
+// with a wavefront each hide their chains behind one another, and the
+// workgroups' barriers only cost: heavy-tailed subgames' leaf input per wave, on
+// workgroups against single wavefronts, with 2,300 + 2,000 long lists of the two
+// players 8.2 against 11.8 ms, 3,200 + 2,700 11.0 against 12.6, 5,300 + 3,900
+// 16.3 against 15.3, 21,800 + 18,100 69.9 against 60.6.
+constexpr uint32_t POOL_LONG = 192, POOL_CH = 64, POOL_FILL = 16;
 // A chunk's reach rows in LDS: config c of a row at POOL_Q (c % 4) + c / 4, so
 // that a lane's configs of four consecutive MFMA steps are one 16-byte read;
 // the pitches spread a wavefront's reads and writes over the banks.
@@ -697,7 +706,7 @@ __device__ __forceinline__ float pool_mass(float tpart, uint32_t q, float (&tot)
     return ti;
 }
 
-// A short list: one wavefront.
+// A list on one wavefront.
 template <int PREC>
 __device__ __forceinline__ void pool_short(const WaveDev& w, const PoolGroup* grp, uint32_t p, uint16_t* x0,
                                            uint16_t* x1, uint16_t (*dst)[POOL_OUT]) {
@@ -767,7 +776,7 @@ __device__ __forceinline__ void pool_short(const WaveDev& w, const PoolGroup* gr
     }
 }
 
-// A long list: the workgroup, one 16-dimension tile per wavefront.
+// A list on the workgroup, one 16-dimension tile per wavefront.
 template <int PREC>
 __device__ __forceinline__ void pool_long(const WaveDev& w, const PoolGroup* grp, uint32_t p, uint16_t* x0,
                                           uint16_t* x1, PoolLds& sh) {
@@ -875,10 +884,10 @@ __global__ __launch_bounds__(BLOCK, 4) void k_pool_mfma(WaveDev w, int player, u
     pool_short<PREC>(w, w.pool_grp[p] + g, p, x0, x1, sh.out[wave][0]);
 }
 
-uint32_t pool_long_groups(const PoolGroup* grp, uint32_t n) {
+uint32_t pool_long_groups(const PoolGroup* grp, uint32_t n, uint32_t cus) {
     uint32_t k = 0;
     while (k < n && grp[k].n > POOL_LONG) k++;
-    return k;
+    return k <= POOL_FILL * cus ? k : 0;
 }
 
 void launch_pool(const WaveDev& w, int player, int precision, void* x0, void* x1, hipStream_t s, int acc,
