@@ -1014,7 +1014,14 @@ __device__ __forceinline__ void backprop_row(const WaveDev& w, int p, BackRec q,
     // predict delta, EPS), normalised by a reciprocal multiply. The sum's
     // discount (sum *= ds) is taken with the accumulation in the reach sweep.
     const float* st = MODE == MODE_VALUE ? strat : w.cur;
-    if (n - 1 < ROW_BATCH) {  // 1 to 12 actions: everything stays in registers
+    // A config without actions has the value zero and owns no cell. (Leaving here
+    // costs nothing; bounding the branch below to 1 to 12 actions instead, the
+    // heavy-tailed wave's CFR passes took 111.7 ms for 110.5.)
+    if (n == 0) {
+        put(q.out, 0.0f);
+        return;
+    }
+    if (n <= ROW_BATCH) {  // everything stays in registers
         uint32_t lvi[ROW_QUADS][4];
         float sv[ROW_QUADS][4], qv[ROW_QUADS][4], old[ROW_QUADS][4];
         const bool more[ROW_QUADS] = {true, n > 4, n > 8};
@@ -1073,8 +1080,7 @@ __device__ __forceinline__ void backprop_row(const WaveDev& w, int p, BackRec q,
         return;
     }
     // Longer rows: the same arithmetic in three batched passes (base; update,
-    // with cur holding the unnormalised value; normalisation). A config without
-    // actions comes here too: it owns no cell, and no pass reads or writes one.
+    // with cur holding the unnormalised value; normalisation).
     float base = 0.0f;
     for (uint32_t c0 = 0; c0 < n; c0 += ROW_BATCH) {
         const uint32_t m = n - c0 < ROW_BATCH ? n - c0 : ROW_BATCH;
