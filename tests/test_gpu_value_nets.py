@@ -178,6 +178,46 @@ def test_compensated_fused_net(inputs, hidden, layers, heads, rows, offset):
     assert np.abs(got[:500] - ref).max() <= 1e-5 * np.abs(ref).max()
 
 
+# both sides of the lines: a block per CU and more, heads about as wide as a CU should stream, two rounds of passes
+@pytest.mark.parametrize("inputs,hidden,layers,heads,rows", [
+    (512, 384, 1, 1536, 33), (512, 384, 1, 1540, 33), (96, 64, 2, 1024, 4100), (96, 64, 2, 1030, 4100),
+    (96, 64, 1, 830, 20000), (96, 64, 1, 850, 20000)])
+def test_compensated_net_under_a_wide_head(inputs, hidden, layers, heads, rows):
+    """Planned passes where the fused net pays and layer by layer where it does not, bit for bit the launch from device
+    rows, which is always fused."""
+    say(f"case compensated wide head: {rows} rows, {inputs} -> {layers}x{hidden} -> {heads}")
+    net = ww.synth_weights(ww.mlp_dims(inputs, hidden, layers, heads, pool=8), seed=rows)
+    x = ww.synth_features(rows, inputs, seed=rows + 1)
+    ex = ww.Executor(0, ww.WC_F16X)
+    v = ex.publish(net)
+    got, want = ex.mlp(v, x, heads=heads), forward_on_device(ex, v, x, heads, 0)
+    ex.close()
+    np.testing.assert_array_equal(got, want)
+
+
+@pytest.mark.parametrize("info,fused", [(1500, True), (2000, False)])
+def test_compensated_wave_under_a_wide_head(info, fused):
+    """The same line inside a wave, by the widths its row blocks need: leaf values at the initial reach against the
+    oracle's model of the compensated operands, within the bound of the other probes of this mode."""
+    say(f"case compensated wave: lists of up to {info} configs")
+    dims = ww.mlp_dims(inputs=96, hidden=64, layers=1, heads=info, pool=16)
+    jobs = ww.synth_jobs(dims, seed=info, trees=2, nodes_lo=12, nodes_hi=20, act_lo=2, act_hi=3, collapse=0.2,
+                         chance=1, draw_lo=2, draw_hi=2, info_fixed=info, dirichlet=1, iters=2, depth=2, snapshots=1,
+                         nroots=1, **W.DCFR)
+    net = ww.synth_weights(dims, seed=info + 1)
+    ex = ww.Executor(0, ww.WC_F16X)
+    v = ex.publish(net)
+    wave = ww.Wave(jobs)
+    for p in (0, 1):
+        widest = int(wave.array(f"head_rb_n{p}").max())
+        assert (widest <= 1536) == fused and widest > 1024
+        got, _ = ex.leaf_probe(wave, v, p)
+        want = np.concatenate([O.leaf_probe(j, net, O.NET_F16X, p)[0] for j in jobs])
+        assert np.abs(got - want).max() <= 1e-5 * np.abs(want).max()
+    wave.close()
+    ex.close()
+
+
 # idle wavefronts, one to four feature blocks each, one to three layers; few rows and several blocks per pass
 @pytest.mark.parametrize("precision,mode,bound", [(ww.WC_F16, O.NET_F16, 2e-3), (ww.WC_BF16, O.NET_BF16, 1e-2)])
 @pytest.mark.parametrize("inputs,width,layers,trees,nodes", [

@@ -525,6 +525,7 @@ bool Executor::upload(const WaveHost& w, const NetBank& bank, uint32_t slot, std
     o.unit_term = blob.put(w.unit_term);
     o.head_tile_n = blob.put(w.head_tile_n);
     std::vector<ChainPass> plan[2];
+    bool fuse[2];
     for (int p = 0; p < 2; p++) {
         plan[p] = plan_chain(w.head_rb_n[p].data(), (uint32_t)w.head_rb_n[p].size(), w.net.heads, cus_,
                              chain_most(precision_));
@@ -533,6 +534,13 @@ bool Executor::upload(const WaveHost& w, const NetBank& bank, uint32_t slot, std
         o.hb[p] = blob.put(w.head_rb_n[p]);
         o.cp[p] = blob.put(plan[p]);
         chain_npass_[p] = (uint32_t)plan[p].size();
+        uint32_t widest = 0;
+        uint64_t columns = 0;
+        for (uint32_t n : w.head_rb_n[p]) {
+            widest = std::max(widest, n);
+            columns += n;
+        }
+        fuse[p] = chain_pays(precision_, (uint32_t)w.head_rb_n[p].size(), widest, columns, cus_);
     }
     for (int p = 0; p < 2; p++) {
         o.tb[p] = blob.put(w.top_back_rec[p]);
@@ -655,7 +663,7 @@ bool Executor::upload(const WaveHost& w, const NetBank& bank, uint32_t slot, std
     d.unit_term = (const uint32_t*)(T + o.unit_term);
     head_tile_n_ = (const uint32_t*)(T + o.head_tile_n);
     for (int p = 0; p < 2; p++) {
-        chain_plan_[p] = (const ChainPass*)(T + o.cp[p]);
+        chain_plan_[p] = fuse[p] ? (const ChainPass*)(T + o.cp[p]) : nullptr;
         head_rb_n_[p] = (const uint32_t*)(T + o.hb[p]);
     }
     for (int p = 0; p < 2; p++) {
@@ -823,7 +831,7 @@ void Executor::run_mlp(const NetBank& bank, uint32_t rows, const void* x, std::v
             marks->push_back(e);
         }
     };
-    if (precision_ != WC_PRECISE && chain_fits(ns.in, ns.hidden, ns.layers)) {
+    if (plan && chain_fits(ns.in, ns.hidden, ns.layers)) {
         ChainNet net = chain_net(bank);
         net.xplane = size_t(gemm_rows(rows)) * ns.in;
         if (part) {
@@ -1561,7 +1569,9 @@ bool Executor::mlp_forward(uint64_t version, uint32_t rows, const float* x, floa
     H_[1] = M + m_h1;
     S_[0] = S_[1] = nullptr;  // this layout holds no partial products
     head_out_ = (float*)(M + m_out);
-    mlp_plan_ = (const ChainPass*)(M + m_plan);
+    const uint32_t nrb = (rows + 15) / 16;
+    mlp_plan_ = chain_pays(precision_, nrb, ns.heads, uint64_t(nrb) * ns.heads, cus_) ? (const ChainPass*)(M + m_plan)
+                                                                                     : nullptr;
     mlp_npass_ = (uint32_t)plan.size();
     if (!plan.empty())
         HIP_TRY(hipMemcpyAsync(M + m_plan, plan.data(), plan.size() * sizeof(ChainPass), hipMemcpyHostToDevice,

@@ -274,7 +274,8 @@ class Executor {
     const uint32_t* head_tile_n_ = nullptr;  // head width per 128-row tile (device copy)
     bool built_ = false;  // the uploaded wave's v5 build is queued already; the next schedule leaves it out
     const uint32_t* head_rb_n_[2] = {};      // head width per 16-row block and traverser (device copies)
-    const ChainPass* chain_plan_[2] = {};    // fused value net passes per traverser (device copies)
+    // fused value net passes per traverser (device copies); null where the net runs layer by layer
+    const ChainPass* chain_plan_[2] = {};
     uint32_t chain_npass_[2] = {0, 0};
     const ChainPass* mlp_plan_ = nullptr;    // the same for mlp_forward's rows
     uint32_t mlp_npass_ = 0;

@@ -184,6 +184,9 @@ struct ChainNet {
 // Blocks a pass holds: a compensated operand takes twice the LDS.
 uint32_t chain_most(int precision);
 bool chain_fits(uint32_t in, uint32_t hidden, uint32_t layers);
+// Whether the fused net is the faster one for nrb row blocks of a shape that
+// fits, the widest needing `widest` head columns and all together `columns`.
+bool chain_pays(int precision, uint32_t nrb, uint32_t widest, uint64_t columns, uint32_t cus);
 void launch_chain(int precision, const ChainNet& net, const void* X, uint32_t rows, float* out,
                   const ChainPass* plan, uint32_t npass, hipStream_t s);
 // The whole network over rows that all need the whole head, from a row-major

@@ -1811,6 +1811,21 @@ bool chain_fits(uint32_t in, uint32_t hidden, uint32_t layers) {
 
 uint32_t chain_most(int precision) { return precision == WC_F16X ? CHAIN_PASS_BLOCKS / 2 : CHAIN_PASS_BLOCKS; }
 
+// A compensated pass streams its head, both planes, from L2 for at most four
+// row blocks, where the layer-by-layer product's tiles share it over 128 rows:
+// under a wide head the fused net loses what its trunk gains. The line is on the
+// columns a CU streams: the widest block's, or four blocks at a time its share
+// of all. Fused against layer by layer, shapes of one to three layers 64 to 384
+// wide (us): 4,000 rows with 567 heads 31 against 73 and with 1,000 39 against
+// 65; 12,000 rows with 1,000 heads 115 against 111 and with 2,000 196 against
+// 147; 30,000 rows with 768 heads 1.1 to 1.4 times as long; up to a block per CU
+// even at about 1,500 to 2,000 heads (a row, 4,000 heads: 85 against 35).
+bool chain_pays(int precision, uint32_t nrb, uint32_t widest, uint64_t columns, uint32_t cus) {
+    if (precision != WC_F16X) return precision != WC_PRECISE;
+    const uint64_t streamed = std::max<uint64_t>(widest, columns / (CHAIN_PASS_BLOCKS / 2 * cus));
+    return streamed <= (nrb <= cus ? 1536 : 1024);
+}
+
 template <int PREC>
 __device__ __forceinline__ float4v mfma16(const uint4& a, const uint4& b, const float4v& c) {
     if (PREC == WC_F16)
