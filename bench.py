@@ -195,7 +195,7 @@ def main():
         if mlp_ms > 0 else 0.0
     # The roofline names one kernel: the one with the most device time per wave
     # among the subtree sweep, the subtree reach and the value net.
-    net_name = "two-tower net (k_gemm layers + k_tower_dense)" if tower else "k_chain"
+    net_name = "two-tower net (k_tower, private k_gemm layers, k_tower_dense)" if tower else "k_chain"
     per_wave = {"k_sweep<regret>": back_ms * iters, "k_reach": reach_ms * iters, net_name: mlp_ms}
     dominant = max(per_wave, key=per_wave.get)
     if dominant == net_name:
